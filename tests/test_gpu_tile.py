@@ -1,0 +1,64 @@
+"""The 128-row MFMA tile kernel (csrc/tile_gemm.hip) at the edges of its tiles:
+expert row counts around every tile height (multiples of 32 rows), one to nine
+128-k chunks (its chunk buffers are four deep up to 64 rows, two above), K and N
+that leave partial chunks and column tiles, groups of 64 and 128, and more
+tiles than workgroups.
+
+INT4 rows meet the fp32-summation bound of test_gpu_int4_exact; the MXFP4 MLP is
+held to the relative-L2 bound of test_gpu_mxfp4.
+"""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from oracle.torch_ref import moe_mxfp4_ref
+from tests._helpers import softmax_weights
+from tests.test_gpu_int4_exact import _bounded_check, _device_inputs, _gemm_rows
+from xkernels_amd import Backend, _lib, fused_moe_mxfp4, make_mxfp4_moe_weights
+
+pytestmark = pytest.mark.gpu
+
+ROWS = [1, 16, 31, 32, 33, 64, 65, 0, 96, 97, 127, 128, 129, 257]
+
+
+def _row_ids(rows, seed):
+    """top_k = 1 routing with exactly rows[e] tokens on expert e, shuffled."""
+    ids = torch.cat([torch.full((n,), e, dtype=torch.int32) for e, n in enumerate(rows)])
+    return ids[torch.randperm(ids.numel(), generator=torch.Generator().manual_seed(seed))].reshape(-1, 1)
+
+
+@pytest.mark.parametrize("N,K,gs", [(256, 512, 32), (272, 1024, 32), (512, 2048, 32), (256, 1536, 32)]
+                         + [(48, 128 * c, 32) for c in (1, 2, 3, 5, 7, 9)]
+                         + [(304, 32, 32), (256, 96, 32), (256, 160, 32), (256, 640, 64), (528, 1152, 128)])
+def test_int4_tile_edges(N, K, gs, dev):
+    ids = _row_ids(ROWS, K)
+    print(f"int4 tile N={N} K={K} gs={gs}", flush=True)
+    A, packed, scale, ids = _device_inputs(ids.shape[0], len(ROWS), N, K, ids, seed=K + N, gs=gs)
+    # 72 rows per expert on average: the 128-row kernel
+    rows = _gemm_rows(A, packed, scale, ids, flags=_lib._XK_INT4_TEST_FORCE_TILE, gs=gs)
+    assert not torch.isnan(rows).any(), "a routed slot's row was not written"
+    _bounded_check(A, packed, scale, ids, rows, gs=gs)
+
+
+@pytest.mark.parametrize("hidden,ispp", [(512, 512), (1024, 160), (96, 512), (32, 32), (2080, 96), (544, 1536)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_mxfp4_tile_edges(hidden, ispp, dtype, dev):
+    E, M = len(ROWS), sum(ROWS)
+    print(f"mxfp4 tile hidden={hidden} ispp={ispp} {dtype}", flush=True)
+    wts = make_mxfp4_moe_weights(E, hidden, ispp, with_bias=True, device="cpu", seed=hidden, scale_lo=115,
+                                 scale_hi=122)
+    wts["w13_scale"][0, 3, 0] = 255  # the reserved scale code reads as 0
+    wts["w2_scale"][1, 5, 0] = 255
+    A = torch.randn(M, hidden, generator=torch.Generator().manual_seed(1)).to(dtype)
+    ids, w = _row_ids(ROWS, ispp), softmax_weights(M, 1, 3) * 0.7
+    keys = ("w13", "w13_scale", "w2", "w2_scale")
+    got = fused_moe_mxfp4(A.to(dev), *(wts[k].to(dev) for k in keys), ids.to(dev), w.to(dev),
+                          b13=wts["b13"].to(dev), b2=wts["b2"].to(dev), backend=Backend.HIP)
+    want = moe_mxfp4_ref(A, *(wts[k] for k in keys), ids, w, b13=wts["b13"], b2=wts["b2"])
+    assert got.dtype == dtype
+    got, want = got.float().cpu(), want.float()
+    assert torch.isfinite(got).all()
+    # bf16 roundings of the gate/up sums, the activation and the down sums that
+    # fall on other sides of a tie: 2^-9 relative each on a small share of terms
+    assert float((got - want).norm() / want.norm()) < 2e-3

@@ -61,11 +61,17 @@ int topk_softmax_max_experts();
 int launch_topk_softmax(const void* logits, int dtype, int64_t M, int64_t E, int64_t k,
                         int renorm, float* w, int32_t* ids, hipStream_t stream);
 int mxfp4_block_size();
-int launch_mxfp4_stage(int stage, const void* A, int a_dtype, const uint8_t* w,
-                       const uint8_t* ws, const uint16_t* bias, int64_t E, int64_t K,
-                       int64_t rows, int64_t ncols, const int32_t* sorted_ids,
-                       const int32_t* offsets, int64_t numel, int64_t top_k, float limit,
-                       uint16_t* act, float* slot_out, hipStream_t stream);
+int launch_activations_to_bf16(const float* a, int64_t n, uint16_t* out, hipStream_t stream);
+int64_t tile_queue_bytes();
+int launch_clear_queue(int* q, int n, hipStream_t stream);
+int launch_mxfp4_tile(int stage, const uint16_t* A, int64_t a_rows, int64_t K, const uint8_t* w,
+                      const uint8_t* ws, const uint16_t* bias, int64_t E, int64_t rows,
+                      const int32_t* sorted_ids, const int32_t* offsets, int64_t numel,
+                      int64_t a_row_div, float limit, uint16_t* out, int* queue, hipStream_t stream);
+int launch_topk_combine_bf16(const uint16_t* rows, int64_t M, int64_t top_k, int64_t N,
+                             const float* topk_w, int mul_routed_weight, const int32_t* topk_ids,
+                             int num_local, const int32_t* emap, int num_global, void* out,
+                             int out_dtype, hipStream_t stream);
 int mxfp4_rs_slices(int64_t K, int64_t N, int64_t numel, int64_t E);
 bool mxfp4_rs_ok(int64_t a_rows, int64_t K, int64_t N, int64_t E, int64_t numel);
 int launch_mxfp4_rs(const void* A, int64_t a_rows, int64_t K, const uint8_t* w, const uint8_t* ws,
@@ -286,8 +292,8 @@ int xk_moe_int4_w4a16(const void* A, int32_t a_dtype, int64_t M, int64_t K,
     return set_error(XK_ERR_WORKSPACE, "int4: workspace %lld B < %lld B",
                      (long long)workspace_bytes, (long long)need);
   // A batch whose activations the MFMA kernels cannot address (2^31 bytes
-  // through buffer offsets) runs as consecutive token chunks of the largest
-  // size they take: a token's output depends only on its own slots (each slot
+  // through buffer offsets) runs as the fewest even token chunks that they
+  // take: a token's output depends only on its own slots (each slot
   // row is a fixed-order K sum, the combine sums a token's slots in slot
   // order), so the chunks write what one call would, bit for bit, with the
   // MFMA kernels instead of the scalar one. Each chunk lays out its smaller
@@ -297,6 +303,7 @@ int xk_moe_int4_w4a16(const void* A, int32_t a_dtype, int64_t M, int64_t K,
     int64_t mc = ((int64_t(1) << 31) - 1) / (K * elem);
     while (mc > 0 && int4_kernel_code(mc, top_k, E, N, K, a_dtype, group_size, 0, 0) == 0) mc /= 2;
     if (mc > 0 && mc < M) {
+      mc = cdiv(M, cdiv(M, mc));  // even parts: a short last one would take another kernel's summation order
       for (int64_t m0 = 0; m0 < M; m0 += mc) {
         const int64_t mm = std::min(mc, M - m0);
         if (int rc = xk_moe_int4_w4a16(static_cast<const char*>(A) + m0 * K * elem, a_dtype, mm, K,
@@ -405,29 +412,30 @@ int xk_moe_topk_softmax(const void* gating_output, int32_t dtype, int64_t M, int
 namespace {
 
 // The MXFP4 pipeline: both projections through the stream kernel (bf16
-// activations, shapes within its limits), else the per-stage kernels.
-// Workspace after the align scratch: act [numel, ispp] bf16, then the down
-// projection's rows [S1, numel, hidden] fp32, then (stream path) the gate/up
-// planes [S0, numel, 2 ispp] fp32. The slice counts depend on K only, so the
-// workspace bytes never decrease with M and a workspace sized for a batch
-// serves every smaller one.
-int64_t max_plane_rows(int64_t K, int64_t N, int64_t numel, int64_t E) {
-  return mxfp4_rs_slices(K, N, numel, E) * numel;
-}
-
+// activations, few routed rows per expert, shapes within its limits), else
+// through the tile kernel.
+// Workspace after the align scratch: act [numel, ispp] bf16, then the stream
+// path's down planes [S1, numel, hidden] fp32 and gate/up planes [S0, numel,
+// 2 ispp] fp32, or the tile path's down rows [numel, hidden] bf16, its bf16
+// activations [M, hidden] (fp32 calls) and its two tile queues.
+// Routed rows per expert (on average) from which the tile kernel runs: E = 256,
+// hidden 4096, ispp 512, top_k 6, stream vs tile 288 vs 322 us at 14 rows, 400
+// vs 343 at 23; E = 64, hidden 2048, ispp 1408, top_k 8: 123 vs 173 at 19 rows,
+// 226 vs 193 at 50.
 constexpr int64_t kMxStreamRowsPerExpert = 20;
+
+// Whether a batch's activations fit one tile launch (2^31-byte buffers).
+bool mxfp4_tile_fits(int64_t M, int64_t top_k, int64_t hidden, int64_t ispp) {
+  return M * hidden * 2 < (int64_t(1) << 31) && M * top_k * ispp * 2 < (int64_t(1) << 31);
+}
 
 struct Mxfp4Plan {
   bool stream;
   int s0, s1;
-  int64_t act, down, gu, total;
+  int64_t act, down, gu, abf, queue, total;
   Mxfp4Plan(int64_t M, int64_t top_k, int64_t E, int64_t hidden, int64_t ispp, int a_dtype) {
     const int64_t numel = M * top_k;
     AlignScratch al(numel, int(E), mxfp4_block_size());
-    // the stream kernels take each expert's weights once per 16-row pass; from
-    // ~20 routed rows per expert on average the per-stage kernels (32 rows a
-    // pass) are faster (E = 256, hidden 4096, ispp 512: 280.7 vs 338.2 us at
-    // 12 rows per expert, 464.6 vs 445.8 us at 24)
     stream = a_dtype == XK_DT_BF16 && numel > 0 && numel < kMxStreamRowsPerExpert * E &&
              mxfp4_rs_ok(M, hidden, 2 * ispp, E, numel) &&
              mxfp4_rs_ok(numel, ispp, hidden, E, numel);
@@ -435,10 +443,18 @@ struct Mxfp4Plan {
     s1 = stream ? mxfp4_rs_slices(ispp, hidden, numel, E) : 1;
     act = al.total;
     down = act + round_up(numel * ispp * 2);
-    gu = down + round_up((stream ? max_plane_rows(ispp, hidden, numel, E) : numel) * hidden * 4);
-    total = gu + round_up(stream ? max_plane_rows(hidden, 2 * ispp, numel, E) * 2 * ispp * 4 : 0);
+    gu = down + round_up(stream ? s1 * numel * hidden * 4 : numel * hidden * 2);
+    abf = gu;
+    queue = abf + round_up(stream || a_dtype == XK_DT_BF16 ? 0 : M * hidden * 2);
+    total = stream ? gu + round_up(s0 * numel * 2 * ispp * 4) : queue + round_up(2 * tile_queue_bytes());
   }
 };
+
+// Tokens of the largest part of a batch that one tile launch takes.
+int64_t mxfp4_tile_tokens(int64_t M, int64_t top_k, int64_t hidden, int64_t ispp) {
+  while (M > 1 && !mxfp4_tile_fits(M, top_k, hidden, ispp)) M = (M + 1) / 2;
+  return M;
+}
 
 }  // namespace
 
@@ -446,9 +462,13 @@ extern "C" {
 
 int64_t xk_moe_mxfp4_workspace_bytes(int64_t M, int64_t top_k, int64_t E, int64_t hidden,
                                      int64_t ispp) {
-  // the larger of the two plans (the activation dtype is not an argument)
-  return std::max(Mxfp4Plan(M, top_k, E, hidden, ispp, XK_DT_BF16).total,
-                  Mxfp4Plan(M, top_k, E, hidden, ispp, XK_DT_FP32).total);
+  // the larger of the two dtypes' plans (the dtype is not an argument), and of
+  // the largest batch below this one that the stream path may take: a workspace
+  // sized for a batch serves every smaller one
+  const int64_t below = std::min(M, (kMxStreamRowsPerExpert * E - 1) / std::max<int64_t>(top_k, 1));
+  return std::max({Mxfp4Plan(M, top_k, E, hidden, ispp, XK_DT_BF16).total,
+                   Mxfp4Plan(M, top_k, E, hidden, ispp, XK_DT_FP32).total,
+                   Mxfp4Plan(below, top_k, E, hidden, ispp, XK_DT_BF16).total});
 }
 
 int xk_moe_mxfp4(const void* A, int32_t a_dtype, int64_t M, int64_t hidden, const uint8_t* w13,
@@ -473,11 +493,26 @@ int xk_moe_mxfp4(const void* A, int32_t a_dtype, int64_t M, int64_t hidden, cons
   if (workspace == nullptr || workspace_bytes < need)
     return set_error(XK_ERR_WORKSPACE, "mxfp4: workspace %lld B < %lld B",
                      (long long)workspace_bytes, (long long)need);
+  const Mxfp4Plan plan(M, top_k, E, hidden, ispp, a_dtype);
+  if (!plan.stream && !mxfp4_tile_fits(M, top_k, hidden, ispp)) {
+    // a batch whose activations reach 2^31 bytes runs as consecutive token
+    // chunks (a token's output depends only on its own slots); each lays out
+    // its smaller workspace at the start of this one
+    const int64_t mc = mxfp4_tile_tokens(M, top_k, hidden, ispp);
+    XK_REQUIRE(mxfp4_tile_fits(mc, top_k, hidden, ispp), "mxfp4: one token's activations reach 2^31 bytes");
+    const int64_t elem = a_dtype == XK_DT_FP32 ? 4 : 2;
+    for (int64_t m0 = 0; m0 < M; m0 += mc)
+      if (int rc = xk_moe_mxfp4(static_cast<const char*>(A) + m0 * hidden * elem, a_dtype, std::min(mc, M - m0),
+                                hidden, w13, w13_scale, w2, w2_scale, E, ispp, b13, b2, swiglu_limit, group_size,
+                                topk_ids + m0 * top_k, topk_w != nullptr ? topk_w + m0 * top_k : nullptr, top_k,
+                                expert_map, num_global_experts, mul_routed_weight,
+                                static_cast<char*>(out) + m0 * hidden * elem, workspace, workspace_bytes, stream))
+        return rc;
+    return XK_OK;
+  }
   const int64_t numel = M * top_k;
   AlignScratch al(numel, int(E), mxfp4_block_size());
-  const Mxfp4Plan plan(M, top_k, E, hidden, ispp, a_dtype);
   uint16_t* act = at<uint16_t>(workspace, plan.act);
-  float* slot_out = at<float>(workspace, plan.down);
   int32_t* sorted = at<int32_t>(workspace, al.sorted);
   int32_t* offsets = at<int32_t>(workspace, al.offsets);
   // the stream kernels route small batches themselves (no align kernel)
@@ -494,6 +529,7 @@ int xk_moe_mxfp4(const void* A, int32_t a_dtype, int64_t M, int64_t hidden, cons
     const int32_t* rs_sorted = self_route ? nullptr : sorted;
     const int32_t* rs_offsets = self_route ? nullptr : offsets;
     float* gu = at<float>(workspace, plan.gu);
+    float* slot_out = at<float>(workspace, plan.down);
     rc = launch_mxfp4_rs(A, M, hidden, w13, w13_scale, E, 2 * ispp, numel, top_k, rs_sorted,
                          rs_offsets, topk_ids, expert_map, num_global_experts, gu, stream);
     if (rc) return rc;
@@ -507,14 +543,24 @@ int xk_moe_mxfp4(const void* A, int32_t a_dtype, int64_t M, int64_t hidden, cons
                                int(E), expert_map, num_global_experts, out, a_dtype, plan.s1, stream,
                                b2, 1);
   }
-  rc = launch_mxfp4_stage(0, A, a_dtype, w13, w13_scale, b13, E, hidden, 2 * ispp, ispp, sorted,
-                          offsets, numel, top_k, swiglu_limit, act, nullptr, stream);
+  const uint16_t* a16 = static_cast<const uint16_t*>(A);
+  if (a_dtype == XK_DT_FP32) {
+    uint16_t* abf = at<uint16_t>(workspace, plan.abf);
+    if ((rc = launch_activations_to_bf16(static_cast<const float*>(A), M * hidden, abf, stream))) return rc;
+    a16 = abf;
+  }
+  uint16_t* rows = at<uint16_t>(workspace, plan.down);
+  int* queue = at<int>(workspace, plan.queue);
+  const int nq = int(tile_queue_bytes() / sizeof(int));
+  if ((rc = launch_clear_queue(queue, 2 * nq, stream))) return rc;
+  rc = launch_mxfp4_tile(0, a16, M, hidden, w13, w13_scale, b13, E, 2 * ispp, sorted, offsets, numel, top_k,
+                         swiglu_limit, act, queue, stream);
   if (rc) return rc;
-  rc = launch_mxfp4_stage(1, act, XK_DT_BF16, w2, w2_scale, b2, E, ispp, hidden, hidden, sorted,
-                          offsets, numel, top_k, 0.f, nullptr, slot_out, stream);
+  rc = launch_mxfp4_tile(1, act, numel, ispp, w2, w2_scale, b2, E, hidden, sorted, offsets, numel, 1, 0.f, rows,
+                         queue + nq, stream);
   if (rc) return rc;
-  return launch_topk_combine(slot_out, M, top_k, hidden, topk_w, mul_routed_weight, topk_ids,
-                             int(E), expert_map, num_global_experts, out, a_dtype, 1, stream);
+  return launch_topk_combine_bf16(rows, M, top_k, hidden, topk_w, mul_routed_weight, topk_ids, int(E), expert_map,
+                                  num_global_experts, out, a_dtype, stream);
 }
 
 }  // extern "C"

@@ -10,8 +10,9 @@
 // weighted top-k combine runs afterwards (reduce.hip). Kernels:
 //   * int4_stream_rne (int4_stream.hip): decode regime, bf16 A, group 32 —
 //     weight streaming with the exact bf16 dequant, K-slice partial planes;
-//   * int4_prefill_tile (int4_prefill.hip): prefill regime (>= 17 routed rows
-//     per expert on average), MFMA tiles, the same exact dequant;
+//   * moe_tile (tile_gemm.hip) and int4_prefill_gemm (int4_prefill.hip): prefill
+//     regime (>= 17 routed rows per expert on average), MFMA tiles of 128 and
+//     256 rows, the same exact dequant;
 //   * int4_simple_gemm (below): any dtype, group size or shape the MFMA
 //     kernels do not take — one thread per (slot, column), exact dequant
 //     rounded to A's dtype like the reference.
@@ -95,27 +96,47 @@ int launch_int4_rs(const void* A, bool f32a, int64_t M, int64_t K, const int32_t
                    int group_size, const int32_t* sorted_ids, const int32_t* offsets,
                    const int32_t* topk_ids, const int32_t* emap, int num_global, float* slot_out,
                    hipStream_t stream);
+bool int4_tile_ok(int a_dtype, int group_size, int64_t M, int64_t K, int64_t N, int64_t E);
+int launch_int4_tile(const void* A, int64_t K, const int32_t* packed, const uint16_t* scale,
+                     int64_t E, int64_t N, int64_t numel, int64_t top_k, int group_size,
+                     const int32_t* sorted_ids, const int32_t* offsets, float* slot_out,
+                     int* queue, hipStream_t stream);
 int launch_int4_prefill(const void* A, int64_t K, const int32_t* packed, const uint16_t* scale,
                         int64_t E, int64_t N, int64_t numel, int64_t top_k, int group_size,
                         const int32_t* sorted_ids, const int32_t* offsets, float* slot_out,
                         int* queue, hipStream_t stream);
 
-// Routed rows per expert (on average) from which the tile kernel replaces the
+// Routed rows per expert (on average) from which the tile kernels replace the
 // weight-streaming kernel, which streams every expert's weights once per
-// 16-row pass. Measured at E = 48, N = 4096, K = 7168, top_k = 8 (uniform
-// routing): stream vs tile 177.2 vs 248.4 us at 13.3 rows per expert, 228.9
-// vs 248.1 us at 16, 264.4 vs 249.8 us at 18.7, 294.6 vs 249.2 us at 21.3.
+// 16-row pass. Measured per fused call, stream vs tile (moe_tile), uniform
+// routing: E = 48, N = 4096, K = 7168, top_k = 8: 172 vs 217 us at 10.7 rows
+// per expert, 191 vs 218 at 13.3, 244 vs 221 at 16.7, 311 vs 226 at 21.7, 483
+// vs 256 at 42; N = 7168, K = 2048: 150 vs 165 at 21.7, 360 vs 217 at 67.
 constexpr int64_t kPrefillRowsPerExpert = 17;
+// K or N not a multiple of 256: the tile pads both, the stream kernel little (E =
+// 48, N = K = 2880, top_k = 4: 143 vs 148 us at 33 rows, 175 vs 174 at 83).
+constexpr int64_t kPaddedTileRowsPerExpert = 32;
+
+// The 256-row tile kernel (int4_prefill_gemm) in place of the 128-row one
+// (moe_tile), by routed rows per expert: where most experts fill one 256-row
+// tile but need two of 128 rows, and in batches of several 256-row tiles per
+// expert, where its one dequant per 256 rows saves about 1 %. Per fused call at
+// N = 4096, K = 7168, 256- vs 128-row: 407 vs 343 us at 100 rows, 492 vs 517 at
+// 133, 549 vs 610 at 167, 655 vs 663 at 217, 900 vs 852 at 267, 1,043 vs 965 at
+// 333, 1,388 vs 1,347 at 500, 1,858 vs 1,877 at 683.
+bool int4_tall_tiles(int64_t rows, int64_t E) {
+  return (rows >= 120 * E && rows < 224 * E) || rows >= 600 * E;
+}
 
 // The INT4 kernels need no workspace; the argument and this size stay in the
 // interface (0 bytes, NULL accepted).
-int64_t int4_prefill_queue_bytes();
+int64_t tile_queue_bytes();
 
 // The tile kernel's queue; the other kernels need none.
 int64_t int4_gemm_workspace_bytes(int64_t M, int64_t K) {
   (void)M;
   (void)K;
-  return int4_prefill_queue_bytes();
+  return tile_queue_bytes();
 }
 
 // The grouped-GEMM kernel a call runs, from its shapes and flags only (not
@@ -128,15 +149,18 @@ enum class Int4Kernel { kSimple, kRs, kTile };
 // dense call (numel * E / ep_global slots expected on the local experts), so
 // that an expert-parallel rank picks the kernel the dense call picks for the
 // same rows per expert. 0: every slot counts against the E experts.
+int64_t int4_local_slots(int64_t numel, int64_t E, int64_t ep_global) {
+  return ep_global > E ? (numel * E + ep_global - 1) / ep_global : numel;
+}
 Int4Kernel int4_choose(int64_t M, int64_t top_k, int64_t E, int64_t N, int64_t K, int a_dtype,
                        int group_size, int flags, int64_t ep_global) {
   if (!int4_use_stream(a_dtype, group_size, K)) return Int4Kernel::kSimple;
-  const int64_t numel = M * top_k;
-  const int64_t local = ep_global > E ? (numel * E + ep_global - 1) / ep_global : numel;
+  const int64_t local = int4_local_slots(M * top_k, E, ep_global);
   const bool f32a = a_dtype == XK_DT_FP32;
-  const bool tile_ok = !f32a && int4_prefill_ok(a_dtype, group_size, M, K, N, E);
+  const bool tile_ok = !f32a && int4_tile_ok(a_dtype, group_size, M, K, N, E);
   const bool rs_ok = int4_rs_ok(M, top_k, K, N, E, f32a, group_size);
-  bool tile = tile_ok && local >= kPrefillRowsPerExpert * E;
+  const int64_t from = K % 256 == 0 && N % 256 == 0 ? kPrefillRowsPerExpert : kPaddedTileRowsPerExpert;
+  bool tile = tile_ok && local >= from * E;
   if (flags & XK_INT4_TEST_FORCE_TILE) tile = tile_ok;
   if (flags & XK_INT4_TEST_FORCE_STREAM) tile = tile && !rs_ok;
   if (tile) return Int4Kernel::kTile;
@@ -189,29 +213,38 @@ int launch_int4_gemm(const void* A, int a_dtype, int64_t M, int64_t K, const int
   const int64_t numel = M * top_k;
   XK_REQUIRE(numel < (int64_t(1) << 30), "int4: M*top_k too large");
   if (numel == 0) return XK_OK;
-  const Int4Kernel kern = int4_choose(M, top_k, E, N, K, a_dtype, group_size, flags, ep_global);
+  Int4Kernel kern = int4_choose(M, top_k, E, N, K, a_dtype, group_size, flags, ep_global);
   // the decode kernel routes for itself when no align outputs are given
   const bool self_route = kern == Int4Kernel::kRs && sorted_ids == nullptr && offsets == nullptr &&
                           int4_rs_self_route_ok(numel);
+  const bool aligned = reinterpret_cast<uintptr_t>(A) % 16 == 0 &&
+                       reinterpret_cast<uintptr_t>(packed) % 16 == 0 &&
+                       reinterpret_cast<uintptr_t>(scale) % 16 == 0;
+  // pointers of any alignment run the scalar kernel at sizes that only the tile
+  // kernel of all MFMA kernels takes and that are not multiples of 256 (more
+  // than 512 experts, or a batch past the stream kernel's buffer reach)
+  if (kern == Int4Kernel::kTile && !aligned && !(K % 256 == 0 && N % 256 == 0) &&
+      !int4_rs_ok(M, top_k, K, N, E, false, group_size))
+    kern = Int4Kernel::kSimple;
   if (kern != Int4Kernel::kSimple) {
     XK_REQUIRE(self_route || (sorted_ids && offsets),
                "int4: the MFMA kernels need the align outputs");
-    XK_REQUIRE(reinterpret_cast<uintptr_t>(A) % 16 == 0 &&
-                   reinterpret_cast<uintptr_t>(packed) % 16 == 0 &&
-                   reinterpret_cast<uintptr_t>(scale) % 16 == 0,
-               "int4: A, packed weights and scales must be 16-byte aligned");
+    XK_REQUIRE(aligned, "int4: A, packed weights and scales must be 16-byte aligned");
   }
   switch (kern) {
-    case Int4Kernel::kTile:
+    case Int4Kernel::kTile: {
+      const bool tall = int4_tall_tiles(int4_local_slots(numel, E, ep_global), E) &&
+                        int4_prefill_ok(a_dtype, group_size, M, K, N, E);
       // the tile queue lives in the workspace; without one the tiles are
       // dealt statically
-      return launch_int4_prefill(
+      return (tall ? launch_int4_prefill : launch_int4_tile)(
           A, K, packed, scale, E, N, numel, top_k, group_size, sorted_ids, offsets, slot_out,
-          workspace != nullptr && workspace_bytes >= int4_prefill_queue_bytes() &&
+          workspace != nullptr && workspace_bytes >= tile_queue_bytes() &&
                   reinterpret_cast<uintptr_t>(workspace) % 4 == 0
               ? static_cast<int*>(workspace)
               : nullptr,
           stream);
+    }
     case Int4Kernel::kRs:
       return launch_int4_rs(A, a_dtype == XK_DT_FP32, M, K, packed, scale, E, N, numel, top_k,
                             group_size, sorted_ids, offsets, topk_ids, emap, num_global, slot_out,

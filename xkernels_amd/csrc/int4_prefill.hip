@@ -367,12 +367,6 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& p) {
   }
 }
 
-// Zeroes the tile queue before the tile kernel (a kernel, not a memset, so
-// that a captured graph holds no memset node).
-__global__ void clear_queue(int* q) {
-  if (threadIdx.x < kXcds) q[threadIdx.x] = 0;
-}
-
 __global__ void __launch_bounds__(kPThreads)
 int4_prefill_gemm(PrefillArgs p) {
   prefill_body<false>(p);
@@ -387,8 +381,7 @@ int4_prefill_gemm_g(PrefillArgs p) {
 
 int device_cu_count();
 
-// Bytes of the tile kernel's queue (its workspace).
-int64_t int4_prefill_queue_bytes() { return kXcds * sizeof(int); }
+int launch_clear_queue(int* q, int n, hipStream_t stream);
 
 // Shapes the tile kernel takes: bf16 activations, groups of 32, 64 or 128, K a
 // multiple of two steps, N a multiple of the column tile, at most kPMaxExperts
@@ -409,10 +402,8 @@ int launch_int4_prefill(const void* A, int64_t K, const int32_t* packed, const u
   const int64_t a_bytes = numel / std::max<int64_t>(top_k, 1) * K * 2;
   XK_REQUIRE(a_bytes < (int64_t(1) << 31) && N * K / 2 < (int64_t(1) << 31),
              "int4 prefill: A and one expert's weights must each be below 2^31 bytes");
-  if (queue != nullptr) {
-    hipLaunchKernelGGL(clear_queue, dim3(1), dim3(64), 0, stream, queue);
-    XK_CHECK_LAUNCH("clear_queue");
-  }
+  if (queue != nullptr)
+    if (int rc = launch_clear_queue(queue, kXcds, stream)) return rc;
   PrefillArgs a{static_cast<const uint16_t*>(A), reinterpret_cast<const uint32_t*>(packed), scale,
                 sorted_ids, offsets, slot_out, int(K), int(N), int(numel), int(top_k), int(E),
                 group_size == 128 ? 2 : group_size == 64 ? 1 : 0, queue, int(a_bytes)};

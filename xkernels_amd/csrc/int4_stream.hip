@@ -101,51 +101,6 @@ struct RsArgs {
   int glog;                 // INT4: log2(group size / 32) (GBIG kernels)
 };
 
-// s_waitcnt vmcnt(n) as a real instruction the compiler accounts for (gfx9
-// encoding: vmcnt bits 3:0 and 15:14, expcnt and lgkmcnt left at their maxima).
-#define XK_WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 15) | (((n) >> 4) << 14) | 0x0F70)
-
-// Workgroup barrier that waits for this wave's LDS operations only; the
-// weight loads in flight stay in flight.
-__device__ __forceinline__ void lds_sync() {
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-
-template <typename T> __device__ __forceinline__ T uniform(T x) {
-  return __builtin_amdgcn_readfirstlane(x);
-}
-
-// Buffer descriptor (gfx9 layout: base, num_records, raw 32-bit access) held
-// in SGPRs.
-typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ i32x4 make_rsrc(const void* base, uint32_t bytes) {
-  const uint64_t a = reinterpret_cast<uint64_t>(base);
-  return i32x4{static_cast<int32_t>(uniform(static_cast<uint32_t>(a))),
-               static_cast<int32_t>(uniform(static_cast<uint32_t>(a >> 32))),
-               static_cast<int32_t>(uniform(bytes)), 0x00020000};
-}
-
-// Direct-to-LDS 16-byte buffer load: lane i's 16 bytes from voff + soff land
-// at lds + 16 i. Issued as inline assembly so that the compiler does not make
-// unrelated LDS reads wait for it; the kernel waits for these loads itself
-// (XK_WAIT_VMCNT) before it reads the buffer.
-__device__ __forceinline__ void dma_16(i32x4 rsrc, const void* lds, int voff, int soff) {
-  const uint32_t m0 = uniform(static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds)));
-  asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-               :
-               : "s"(m0), "v"(voff), "s"(rsrc), "s"(uniform(soff))
-               : "memory", "m0");
-}
-
-// f(integral_constant<int, I>) for I = 0 .. N-1: indices that are constants
-// before optimisation, so register arrays indexed by them stay in registers.
-template <int N, typename F, int I = 0> __device__ __forceinline__ void static_for(F&& f) {
-  if constexpr (I < N) {
-    f(std::integral_constant<int, I>{});
-    static_for<N, F, I + 1>(static_cast<F&&>(f));
-  }
-}
-
 // 4 x 4 transpose across the four lanes of a quad (lane bits 0-1 = b):
 // afterwards lane b holds element b of every lane of its quad, in lane order.
 // Two butterfly stages (partners lane ^ 1, then lane ^ 2), one DPP move per

@@ -262,4 +262,18 @@ int launch_topk_combine(const float* slot_out, int64_t M, int64_t top_k, int64_t
                        nparts, pstride);
 }
 
+// The combine of finished bf16 slot rows (the MXFP4 tile path, whose down
+// projection rounds its rows to bf16 and adds the bias itself).
+int launch_topk_combine_bf16(const uint16_t* rows, int64_t M, int64_t top_k, int64_t N,
+                             const float* topk_w, int mul_routed_weight, const int32_t* topk_ids,
+                             int num_local, const int32_t* emap, int num_global, void* out,
+                             int out_dtype, hipStream_t stream) {
+  XK_REQUIRE(top_k >= 1 && top_k <= 1024, "combine: top_k=%lld outside [1, 1024]", (long long)top_k);
+  const RowWeights rw{mul_routed_weight ? topk_w : nullptr, XK_DT_FP32, topk_ids, emap, num_global,
+                      num_local};
+  if (out_dtype == XK_DT_BF16)
+    return launch_reduce(rows, M, int(top_k), N, rw, 1.0f, static_cast<uint16_t*>(out), stream);
+  return launch_reduce(rows, M, int(top_k), N, rw, 1.0f, static_cast<float*>(out), stream);
+}
+
 }  // namespace xk
