@@ -97,3 +97,17 @@ def test_workspace_reuse_smaller_M(dev):
 def test_cpu_tensor_is_rejected():
     with pytest.raises(RuntimeError, match="device tensors"):
         moe_align_block_size(torch.zeros((2, 2), dtype=torch.int32), 4, 4, backend=Backend.HIP)
+
+
+@pytest.mark.parametrize("numel,E", [(2048, 48), (2049, 48), (3072, 8), (4097, 384), (8192, 512), (8193, 1024)])
+def test_grid_path_edges(numel, E, dev):
+    """Slot counts around the one-workgroup path's limit and whole and partial
+    1024-slot chunks, with dropped ids in every chunk; the fused calls' queue
+    clearing rides on the same launches."""
+    print(f"align grid numel={numel} E={E}", flush=True)
+    ids = torch.randint(0, E + 3, (numel, 1), generator=torch.Generator().manual_seed(numel),
+                        dtype=torch.int32)
+    got = moe_align_block_size(ids.to(dev), 16, E, backend=Backend.HIP, truncate=False)
+    want = moe_align_block_size_ref(ids, 16, E, truncate=False)
+    for g, w in zip(got, want):
+        assert torch.equal(g.cpu(), w)

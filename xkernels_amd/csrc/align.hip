@@ -26,6 +26,7 @@ namespace xk {
 namespace {
 
 constexpr int kMaxExperts = 1024;  // local experts (after the EP remap)
+constexpr int64_t kGridChunk = 1024;  // slots per workgroup of the grid path
 
 __device__ __forceinline__ int key_bits(int num_experts) {
   // bits needed to hold keys 0..num_experts (num_experts = the "dropped" key)
@@ -168,8 +169,9 @@ align_single_wg(const int32_t* __restrict__ ids, int64_t numel, int num_experts,
                 int block_size, const int32_t* __restrict__ emap, int num_global,
                 int64_t max_pad, int64_t max_blocks, int32_t* __restrict__ sorted_ids,
                 int32_t* __restrict__ expert_ids, int32_t* __restrict__ num_post,
-                int32_t* __restrict__ expert_offsets) {
+                int32_t* __restrict__ expert_offsets, int* __restrict__ clear, int nclear) {
   extern __shared__ int lds[];
+  if (static_cast<int>(threadIdx.x) < nclear) clear[threadIdx.x] = 0;
   const int nw = blockDim.x >> 6;
   int* cnt = lds;                               // [E]   histogram, then cursor
   int* off = cnt + num_experts;                 // [E+1] padded prefix
@@ -194,8 +196,9 @@ align_single_wg(const int32_t* __restrict__ ids, int64_t numel, int num_experts,
 __global__ void __launch_bounds__(256)
 align_count(const int32_t* __restrict__ ids, int64_t numel, int64_t chunk,
             int num_experts, const int32_t* __restrict__ emap, int num_global,
-            int32_t* __restrict__ chunk_cnt) {
+            int32_t* __restrict__ chunk_cnt, int* __restrict__ clear, int nclear) {
   extern __shared__ int lds[];
+  if (blockIdx.x == 0 && static_cast<int>(threadIdx.x) < nclear) clear[threadIdx.x] = 0;
   for (int i = threadIdx.x; i < num_experts; i += blockDim.x) lds[i] = 0;
   __syncthreads();
   const int64_t begin = blockIdx.x * chunk;
@@ -206,81 +209,99 @@ align_count(const int32_t* __restrict__ ids, int64_t numel, int64_t chunk,
     chunk_cnt[static_cast<int64_t>(blockIdx.x) * num_experts + i] = lds[i];
 }
 
-// Grid phase 2: every workgroup b of 1024 threads
+// Grid phase 2: every workgroup b of 1024 threads, one slot each,
+//   * ranks its slots: the slot's expert loads with the chunk histograms below,
+//     and its rank among the wave's slots of the expert needs no prefix;
 //   * sums the chunk histograms column-wise: total count of every expert and
-//     the count in chunks before b (independent loads, threads (expert, part));
-//   * forms the padded expert prefix (block scan);
-//   * stably scatters its own chunk;
+//     the count in chunks before b (eight independent loads at a time, threads
+//     (expert, part));
+//   * forms the padded expert prefix (block scan) and places its slots;
 //   * writes its 1/nchunks slice of expert_ids and of the pad ids (gap slots of
 //     every expert and the tail), so the layout is written by the whole grid.
 // Workgroup 0 also writes num_tokens_post_padded and expert_offsets.
-__global__ void __launch_bounds__(1024)
-align_place(const int32_t* __restrict__ ids, int64_t numel, int64_t chunk, int nchunks,
+// Bound by the chain of dependent loads and barriers, not by bytes: the slots
+// loaded and ranked after the prefix took 10.0 us at 131,072 slots, this 7.3.
+__global__ void __launch_bounds__(kGridChunk)
+align_place(const int32_t* __restrict__ ids, int64_t numel, int nchunks,
             int num_experts, int block_size, const int32_t* __restrict__ emap,
             int num_global, const int32_t* __restrict__ chunk_cnt, int64_t max_pad,
             int64_t max_blocks, int32_t* __restrict__ sorted_ids,
             int32_t* __restrict__ expert_ids, int32_t* __restrict__ num_post,
             int32_t* __restrict__ expert_offsets) {
   extern __shared__ int lds[];
-  const int nw = blockDim.x >> 6;
+  constexpr int nw = kGridChunk / 64;
   int* tot = lds;                          // [E]   total count of expert e
-  int* base = tot + num_experts;           // [E]   count before this chunk, then cursor
+  int* base = tot + num_experts;           // [E]   first position of this chunk's slots of e
   int* off = base + num_experts;           // [E+1] padded prefix
   int* wsum = off + num_experts + 1;       // [16]
-  int* ctot = wsum + 16;                   // [E]   scatter scratch
-  int* wavecnt = ctot + num_experts;       // [nw][E+1]
+  int* wavecnt = wsum + 16;                // [nw][E+1] slots of e per wave
   int* part = wavecnt + nw * (num_experts + 1);  // [parts][2][E]
-  const int b = blockIdx.x, tid = threadIdx.x;
-  const int parts = max(1, static_cast<int>(blockDim.x) / num_experts);
-  for (int i = tid; i < nw * (num_experts + 1); i += blockDim.x) wavecnt[i] = 0;
+  const int b = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int stride = num_experts + 1;
+  const int64_t t = static_cast<int64_t>(b) * kGridChunk + tid;
+  const int id = t < numel ? ids[t] : -1;
+  const int parts = max(1, static_cast<int>(kGridChunk) / num_experts);
+  for (int i = tid; i < nw * stride; i += kGridChunk) wavecnt[i] = 0;
   {
     // thread (e, p): chunks [p*per, (p+1)*per) of expert e (for e < E when
     // E <= blockDim; otherwise one part and a loop over the experts)
     const int per = static_cast<int>(cdiv(nchunks, parts));
-    for (int idx = tid; idx < parts * num_experts; idx += blockDim.x) {
+    for (int idx = tid; idx < parts * num_experts; idx += kGridChunk) {
       const int e = idx % num_experts, p = idx / num_experts;
       const int b0 = p * per, b1 = min(nchunks, b0 + per);
       int all = 0, before = 0;
-      for (int c = b0; c < b1; ++c) {
-        const int v = chunk_cnt[static_cast<int64_t>(c) * num_experts + e];
-        all += v;
-        before += c < b ? v : 0;
+      for (int c0 = b0; c0 < b1; c0 += 8) {
+        int v[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          v[i] = c0 + i < b1 ? chunk_cnt[static_cast<int64_t>(c0 + i) * num_experts + e] : 0;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          all += v[i];
+          before += c0 + i < b ? v[i] : 0;
+        }
       }
       part[(2 * p) * num_experts + e] = all;
       part[(2 * p + 1) * num_experts + e] = before;
     }
   }
-  __syncthreads();
-  for (int e = tid; e < num_experts; e += blockDim.x) {
-    int all = 0, before = 0;
-    for (int p = 0; p < parts; ++p) {
-      all += part[(2 * p) * num_experts + e];
-      before += part[(2 * p + 1) * num_experts + e];
-    }
-    tot[e] = all;
-    base[e] = before;
+  int key = t < numel ? map_expert(id, emap, num_global, num_experts) : -1;
+  if (key < 0) key = num_experts;
+  uint64_t peers = ~0ull;  // lanes of the same expert
+  for (int i = 0, nbits = key_bits(num_experts); i < nbits; ++i) {
+    const int bit = (key >> i) & 1;
+    const uint64_t bal = __ballot(bit);
+    peers &= bit ? bal : ~bal;
   }
+  const int rank = __popcll(peers & ((lane == 0) ? 0ull : (~0ull >> (64 - lane))));
   __syncthreads();
-  // padded exclusive prefix over experts (num_experts <= blockDim)
-  const int c = tid < num_experts ? tot[tid] : 0;
+  if (rank == 0 && key < num_experts) wavecnt[wave * stride + key] = __popcll(peers);
+  int c = 0, before = 0;
+  if (tid < num_experts)  // num_experts <= blockDim
+    for (int p = 0; p < parts; ++p) {
+      c += part[(2 * p) * num_experts + tid];
+      before += part[(2 * p + 1) * num_experts + tid];
+    }
   const int padded = ((c + block_size - 1) / block_size) * block_size;
   int total = 0;
   const int ex = block_exclusive_scan(padded, wsum, &total);
   if (tid < num_experts) {
+    tot[tid] = c;
     off[tid] = ex;
-    base[tid] += ex;
+    base[tid] = ex + before;
   }
   if (tid == 0) off[num_experts] = total;
   __syncthreads();
+  if (key < num_experts) {
+    int pos = base[key] + rank;
+    for (int w = 0; w < wave; ++w) pos += wavecnt[w * stride + key];
+    sorted_ids[pos] = static_cast<int32_t>(t);
+  }
   if (b == 0) {
     if (tid == 0) num_post[0] = total;
     if (expert_offsets != nullptr)
       for (int e = tid; e <= num_experts; e += blockDim.x) expert_offsets[e] = off[e];
   }
-  // this chunk's slots
-  const int64_t begin = static_cast<int64_t>(b) * chunk;
-  chunk_stable_scatter(ids, begin, min(numel, begin + chunk), emap, num_global, num_experts,
-                       base, wavecnt, ctot, sorted_ids);
   // slice of the layout: expert of a position = #{e in [1, E] : off[e] <= pos}
   auto expert_at = [&](int64_t pos) {
     int lo = 1, hi = num_experts;
@@ -307,27 +328,34 @@ align_place(const int32_t* __restrict__ ids, int64_t numel, int64_t chunk, int n
   }
 }
 
+// One workgroup takes rounds of 1024 slots with five barriers each; the grid
+// path's two launches cost about two rounds more (one workgroup: 8.4 us at 2,000
+// slots, 20.6 us at 6,216). Without the grid path's workspace one workgroup
+// takes up to 8192 slots.
+constexpr int64_t kSingleWgBestSlots = 2048;
 constexpr int64_t kSingleWgMaxSlots = 8192;
 constexpr int kSingleWgMaxExperts = 512;
-constexpr int64_t kGridChunk = 1024;
 
-bool use_single_wg(int64_t numel, int num_experts) {
-  return numel <= kSingleWgMaxSlots && num_experts <= kSingleWgMaxExperts;
+bool use_single_wg(int64_t numel, int num_experts, bool workspace) {
+  return numel <= (workspace ? kSingleWgBestSlots : kSingleWgMaxSlots) && num_experts <= kSingleWgMaxExperts;
 }
 
 }  // namespace
 
 // Bytes of scratch the grid path needs (0 when one workgroup suffices).
 int64_t align_workspace_bytes(int64_t numel, int num_experts) {
-  if (use_single_wg(numel, num_experts)) return 0;
+  if (use_single_wg(numel, num_experts, true)) return 0;
   const int64_t nchunks = std::max<int64_t>(1, cdiv(numel, kGridChunk));
   return nchunks * num_experts * static_cast<int64_t>(sizeof(int32_t));
 }
 
+// `clear`: nclear (at most 64) ints zeroed before the launch's end (a tile
+// kernel's queue: no launch of its own, and no memset in a captured graph).
 int launch_align(const int32_t* ids, int64_t numel, int num_experts, int block_size,
                  const int32_t* emap, int num_global, int32_t* sorted_ids,
                  int32_t* expert_ids, int32_t* num_post, int32_t* expert_offsets,
-                 void* workspace, int64_t workspace_bytes, hipStream_t stream) {
+                 void* workspace, int64_t workspace_bytes, hipStream_t stream, int* clear,
+                 int nclear) {
   XK_REQUIRE(num_experts > 0 && num_experts <= kMaxExperts,
              "align: num_experts=%d outside [1, %d]", num_experts, kMaxExperts);
   XK_REQUIRE(block_size > 0 && block_size <= 4096, "align: block_size=%d outside [1, 4096]",
@@ -339,16 +367,16 @@ int launch_align(const int32_t* ids, int64_t numel, int num_experts, int block_s
   XK_REQUIRE(emap == nullptr || num_global > 0, "align: expert_map needs num_global_experts > 0");
   const int64_t max_pad = numel + static_cast<int64_t>(num_experts + 1) * (block_size - 1);
   const int64_t max_blocks = cdiv(max_pad, block_size);
-  if (use_single_wg(numel, num_experts)) {
+  const int64_t need = align_workspace_bytes(numel, num_experts);
+  if (use_single_wg(numel, num_experts, workspace != nullptr && workspace_bytes >= need)) {
     const int threads = 1024, nw = threads / 64;
     const size_t lds = sizeof(int) * (3 * num_experts + 1 + 16 + nw * (num_experts + 1));
     hipLaunchKernelGGL(align_single_wg, dim3(1), dim3(threads), lds, stream, ids, numel,
                        num_experts, block_size, emap, num_global, max_pad, max_blocks,
-                       sorted_ids, expert_ids, num_post, expert_offsets);
+                       sorted_ids, expert_ids, num_post, expert_offsets, clear, nclear);
     XK_CHECK_LAUNCH("align_single_wg");
     return XK_OK;
   }
-  const int64_t need = align_workspace_bytes(numel, num_experts);
   if (workspace == nullptr || workspace_bytes < need)
     return set_error(XK_ERR_WORKSPACE, "align: workspace %lld B < %lld B",
                      (long long)workspace_bytes, (long long)need);
@@ -356,17 +384,16 @@ int launch_align(const int32_t* ids, int64_t numel, int num_experts, int block_s
   int32_t* chunk_cnt = static_cast<int32_t*>(workspace);
   hipLaunchKernelGGL(align_count, dim3(nchunks), dim3(256), sizeof(int) * num_experts,
                      stream, ids, numel, kGridChunk, num_experts, emap, num_global,
-                     chunk_cnt);
+                     chunk_cnt, clear, nclear);
   XK_CHECK_LAUNCH("align_count");
   {
-    const int threads = 1024, nw = threads / 64;
+    const int threads = kGridChunk, nw = threads / 64;
     const int parts = std::max(1, threads / num_experts);
-    const size_t lds = sizeof(int) * (4 * num_experts + 1 + 16 + nw * (num_experts + 1) +
+    const size_t lds = sizeof(int) * (3 * num_experts + 1 + 16 + nw * (num_experts + 1) +
                                       2 * parts * num_experts);
     hipLaunchKernelGGL(align_place, dim3(nchunks), dim3(threads), lds, stream, ids, numel,
-                       kGridChunk, nchunks, num_experts, block_size, emap, num_global,
-                       chunk_cnt, max_pad, max_blocks, sorted_ids, expert_ids, num_post,
-                       expert_offsets);
+                       nchunks, num_experts, block_size, emap, num_global, chunk_cnt, max_pad,
+                       max_blocks, sorted_ids, expert_ids, num_post, expert_offsets);
     XK_CHECK_LAUNCH("align_place");
   }
   return XK_OK;

@@ -34,7 +34,7 @@ int64_t align_workspace_bytes(int64_t numel, int num_experts);
 int launch_align(const int32_t* ids, int64_t numel, int num_experts, int block_size,
                  const int32_t* emap, int num_global, int32_t* sorted_ids, int32_t* expert_ids,
                  int32_t* num_post, int32_t* expert_offsets, void* workspace,
-                 int64_t workspace_bytes, hipStream_t stream);
+                 int64_t workspace_bytes, hipStream_t stream, int* clear = nullptr, int nclear = 0);
 int launch_sum_reduce(const void* y, int y_dtype, int64_t M, int64_t top_k, int64_t H,
                       const void* w, int w_dtype, float scale, void* out, hipStream_t stream);
 int launch_topk_combine(const float* slot_out, int64_t M, int64_t top_k, int64_t N,
@@ -56,14 +56,13 @@ int launch_int4_gemm(const void* A, int a_dtype, int64_t M, int64_t K, const int
                      const int32_t* topk_ids, int64_t top_k, const int32_t* emap,
                      int num_global, const int32_t* sorted_ids, const int32_t* offsets,
                      float* slot_out, int flags, int64_t ep_global, void* workspace,
-                     int64_t workspace_bytes, hipStream_t stream);
+                     int64_t workspace_bytes, bool queue_cleared, hipStream_t stream);
 int topk_softmax_max_experts();
 int launch_topk_softmax(const void* logits, int dtype, int64_t M, int64_t E, int64_t k,
                         int renorm, float* w, int32_t* ids, hipStream_t stream);
 int mxfp4_block_size();
 int launch_activations_to_bf16(const float* a, int64_t n, uint16_t* out, hipStream_t stream);
 int64_t tile_queue_bytes();
-int launch_clear_queue(int* q, int n, hipStream_t stream);
 int launch_mxfp4_tile(int stage, const uint16_t* A, int64_t a_rows, int64_t K, const uint8_t* w,
                       const uint8_t* ws, const uint16_t* bias, int64_t E, int64_t rows,
                       const int32_t* sorted_ids, const int32_t* offsets, int64_t numel,
@@ -257,7 +256,7 @@ int xk_moe_int4_w4a16_gemm(const void* A, int32_t a_dtype, int64_t M, int64_t K,
   clear_error();
   return launch_int4_gemm(A, a_dtype, M, K, packed, scale, E, N, group_size, topk_ids, top_k,
                           expert_map, num_global_experts, sorted_token_ids, expert_offsets,
-                          slot_out, flags, 0, workspace, workspace_bytes, stream);
+                          slot_out, flags, 0, workspace, workspace_bytes, false, stream);
 }
 
 int xk_moe_topk_combine(const float* slot_out, int64_t M, int64_t top_k, int64_t N,
@@ -346,7 +345,8 @@ int xk_moe_int4_w4a16(const void* A, int32_t a_dtype, int64_t M, int64_t K,
                           at<int32_t>(workspace, al.expert_ids),
                           at<int32_t>(workspace, al.num_post),
                           at<int32_t>(workspace, al.offsets), at<char>(workspace, al.inner),
-                          al.total - al.inner, stream);
+                          al.total - al.inner, stream, at<int>(workspace, al.total),
+                          int(tile_queue_bytes() / sizeof(int)));
     if (rc) return rc;
     sorted = at<int32_t>(workspace, al.sorted);
     offsets = at<int32_t>(workspace, al.offsets);
@@ -354,7 +354,7 @@ int xk_moe_int4_w4a16(const void* A, int32_t a_dtype, int64_t M, int64_t K,
   if (int rc = launch_int4_gemm(A, a_dtype, M, K, packed, scale, E, N, group_size, topk_ids,
                                 top_k, expert_map, num_global_experts, sorted, offsets,
                                 slot_out, flags, ep_global, at<char>(workspace, al.total),
-                                round_up(int4_gemm_workspace_bytes(M, K)), stream))
+                                round_up(int4_gemm_workspace_bytes(M, K)), sorted != nullptr, stream))
     return rc;
   return launch_topk_combine(slot_out, M, top_k, N, topk_w, mul_routed_weight, topk_ids,
                              int(E), expert_map, num_global_experts, out, a_dtype,
@@ -517,12 +517,14 @@ int xk_moe_mxfp4(const void* A, int32_t a_dtype, int64_t M, int64_t hidden, cons
   int32_t* offsets = at<int32_t>(workspace, al.offsets);
   // the stream kernels route small batches themselves (no align kernel)
   const bool self_route = plan.stream && int4_rs_self_route_ok(numel);
+  int* queue = at<int>(workspace, plan.queue);  // the tile path's two
+  const int nq = int(tile_queue_bytes() / sizeof(int));
   int rc = XK_OK;
   if (!self_route) {
     rc = launch_align(topk_ids, numel, int(E), mxfp4_block_size(), expert_map, num_global_experts,
                       sorted, at<int32_t>(workspace, al.expert_ids),
                       at<int32_t>(workspace, al.num_post), offsets, at<char>(workspace, al.inner),
-                      al.total - al.inner, stream);
+                      al.total - al.inner, stream, plan.stream ? nullptr : queue, plan.stream ? 0 : 2 * nq);
     if (rc) return rc;
   }
   if (plan.stream) {
@@ -550,9 +552,6 @@ int xk_moe_mxfp4(const void* A, int32_t a_dtype, int64_t M, int64_t hidden, cons
     a16 = abf;
   }
   uint16_t* rows = at<uint16_t>(workspace, plan.down);
-  int* queue = at<int>(workspace, plan.queue);
-  const int nq = int(tile_queue_bytes() / sizeof(int));
-  if ((rc = launch_clear_queue(queue, 2 * nq, stream))) return rc;
   rc = launch_mxfp4_tile(0, a16, M, hidden, w13, w13_scale, b13, E, 2 * ispp, sorted, offsets, numel, top_k,
                          swiglu_limit, act, queue, stream);
   if (rc) return rc;

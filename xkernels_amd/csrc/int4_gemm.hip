@@ -100,11 +100,11 @@ bool int4_tile_ok(int a_dtype, int group_size, int64_t M, int64_t K, int64_t N, 
 int launch_int4_tile(const void* A, int64_t K, const int32_t* packed, const uint16_t* scale,
                      int64_t E, int64_t N, int64_t numel, int64_t top_k, int group_size,
                      const int32_t* sorted_ids, const int32_t* offsets, float* slot_out,
-                     int* queue, hipStream_t stream);
+                     int* queue, bool queue_cleared, hipStream_t stream);
 int launch_int4_prefill(const void* A, int64_t K, const int32_t* packed, const uint16_t* scale,
                         int64_t E, int64_t N, int64_t numel, int64_t top_k, int group_size,
                         const int32_t* sorted_ids, const int32_t* offsets, float* slot_out,
-                        int* queue, hipStream_t stream);
+                        int* queue, bool queue_cleared, hipStream_t stream);
 
 // Routed rows per expert (on average) from which the tile kernels replace the
 // weight-streaming kernel, which streams every expert's weights once per
@@ -201,7 +201,7 @@ int launch_int4_gemm(const void* A, int a_dtype, int64_t M, int64_t K, const int
                      const int32_t* topk_ids, int64_t top_k, const int32_t* emap,
                      int num_global, const int32_t* sorted_ids, const int32_t* offsets,
                      float* slot_out, int flags, int64_t ep_global, void* workspace,
-                     int64_t workspace_bytes, hipStream_t stream) {
+                     int64_t workspace_bytes, bool queue_cleared, hipStream_t stream) {
   XK_REQUIRE(a_dtype == XK_DT_BF16 || a_dtype == XK_DT_FP32, "int4: bad A dtype %d", a_dtype);
   XK_REQUIRE((flags & ~(XK_INT4_TEST_FORCE_TILE | XK_INT4_TEST_FORCE_STREAM)) == 0,
              "int4: unknown flags 0x%x (pass 0)", flags);
@@ -243,7 +243,7 @@ int launch_int4_gemm(const void* A, int a_dtype, int64_t M, int64_t K, const int
                   reinterpret_cast<uintptr_t>(workspace) % 4 == 0
               ? static_cast<int*>(workspace)
               : nullptr,
-          stream);
+          queue_cleared, stream);
     }
     case Int4Kernel::kRs:
       return launch_int4_rs(A, a_dtype == XK_DT_FP32, M, K, packed, scale, E, N, numel, top_k,

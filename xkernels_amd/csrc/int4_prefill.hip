@@ -396,13 +396,13 @@ bool int4_prefill_ok(int a_dtype, int group_size, int64_t M, int64_t K, int64_t 
 int launch_int4_prefill(const void* A, int64_t K, const int32_t* packed, const uint16_t* scale,
                         int64_t E, int64_t N, int64_t numel, int64_t top_k, int group_size,
                         const int32_t* sorted_ids, const int32_t* offsets, float* slot_out,
-                        int* queue, hipStream_t stream) {
+                        int* queue, bool queue_cleared, hipStream_t stream) {
   XK_REQUIRE(reinterpret_cast<uintptr_t>(A) % 16 == 0 && reinterpret_cast<uintptr_t>(packed) % 16 == 0,
              "int4 prefill: A and packed must be 16-byte aligned");
   const int64_t a_bytes = numel / std::max<int64_t>(top_k, 1) * K * 2;
   XK_REQUIRE(a_bytes < (int64_t(1) << 31) && N * K / 2 < (int64_t(1) << 31),
              "int4 prefill: A and one expert's weights must each be below 2^31 bytes");
-  if (queue != nullptr)
+  if (queue != nullptr && !queue_cleared)
     if (int rc = launch_clear_queue(queue, kXcds, stream)) return rc;
   PrefillArgs a{static_cast<const uint16_t*>(A), reinterpret_cast<const uint32_t*>(packed), scale,
                 sorted_ids, offsets, slot_out, int(K), int(N), int(numel), int(top_k), int(E),

@@ -568,12 +568,12 @@ bool int4_tile_ok(int a_dtype, int group_size, int64_t M, int64_t K, int64_t N, 
 int launch_int4_tile(const void* A, int64_t K, const int32_t* packed, const uint16_t* scale,
                         int64_t E, int64_t N, int64_t numel, int64_t top_k, int group_size,
                         const int32_t* sorted_ids, const int32_t* offsets, float* slot_out,
-                        int* queue, hipStream_t stream) {
+                        int* queue, bool queue_cleared, hipStream_t stream) {
   XK_REQUIRE(reinterpret_cast<uintptr_t>(A) % 16 == 0 && reinterpret_cast<uintptr_t>(packed) % 16 == 0,
              "int4 tile: A and packed must be 16-byte aligned");
   const int64_t a_bytes = numel / std::max<int64_t>(top_k, 1) * K * 2;
   XK_REQUIRE(a_bytes < (int64_t(1) << 31), "int4 tile: A must be below 2^31 bytes");
-  if (queue != nullptr)
+  if (queue != nullptr && !queue_cleared)
     if (int rc = launch_clear_queue(queue, kXcds, stream)) return rc;
   TileArgs a{static_cast<const uint16_t*>(A), reinterpret_cast<const uint8_t*>(packed),
              reinterpret_cast<const uint8_t*>(scale), nullptr, sorted_ids, offsets, slot_out, queue,
