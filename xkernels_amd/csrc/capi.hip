@@ -62,6 +62,18 @@ int launch_topk_softmax(const void* logits, int dtype, int64_t M, int64_t E, int
                         int renorm, float* w, int32_t* ids, hipStream_t stream);
 int mxfp4_block_size();
 int launch_activations_to_bf16(const float* a, int64_t n, uint16_t* out, hipStream_t stream);
+bool small_int4_ok(int a_dtype, int64_t M, int64_t top_k, int64_t E, int64_t N, int64_t K, int group_size,
+                   const void* A, const void* packed, const void* scale);
+int launch_small_int4(const uint16_t* A, int64_t M, int64_t K, const int32_t* packed, const uint16_t* scale,
+                      int64_t E, int64_t N, const int32_t* topk_ids, const float* weights, int64_t top_k,
+                      const int32_t* emap, int num_global, uint16_t* out, hipStream_t stream);
+bool small_mxfp4_ok(int a_dtype, int64_t M, int64_t top_k, int64_t E, int64_t hidden, int64_t ispp, const void* A,
+                    const void* w13, const void* w13_scale, const void* w2, const void* w2_scale);
+int launch_small_mxfp4(const uint16_t* A, int64_t M, int64_t hidden, const uint8_t* w13, const uint8_t* s13,
+                       const uint8_t* w2, const uint8_t* s2, int64_t E, int64_t ispp, const uint16_t* b13,
+                       const uint16_t* b2, float limit, const int32_t* topk_ids, const float* weights,
+                       int64_t top_k, const int32_t* emap, int num_global, uint16_t* act, uint16_t* out,
+                       hipStream_t stream);
 int64_t tile_queue_bytes();
 int launch_mxfp4_tile(int stage, const uint16_t* A, int64_t a_rows, int64_t K, const uint8_t* w,
                       const uint8_t* ws, const uint16_t* bias, int64_t E, int64_t rows,
@@ -290,6 +302,10 @@ int xk_moe_int4_w4a16(const void* A, int32_t a_dtype, int64_t M, int64_t K,
   if (workspace == nullptr || workspace_bytes < need)
     return set_error(XK_ERR_WORKSPACE, "int4: workspace %lld B < %lld B",
                      (long long)workspace_bytes, (long long)need);
+  if (flags == 0 && small_int4_ok(a_dtype, M, top_k, E, N, K, group_size, A, packed, scale))
+    return launch_small_int4(static_cast<const uint16_t*>(A), M, K, packed, scale, E, N, topk_ids,
+                             mul_routed_weight ? topk_w : nullptr, top_k, expert_map, num_global_experts,
+                             static_cast<uint16_t*>(out), stream);
   // A batch whose activations the MFMA kernels cannot address (2^31 bytes
   // through buffer offsets) runs as the fewest even token chunks that they
   // take: a token's output depends only on its own slots (each slot
@@ -494,6 +510,11 @@ int xk_moe_mxfp4(const void* A, int32_t a_dtype, int64_t M, int64_t hidden, cons
     return set_error(XK_ERR_WORKSPACE, "mxfp4: workspace %lld B < %lld B",
                      (long long)workspace_bytes, (long long)need);
   const Mxfp4Plan plan(M, top_k, E, hidden, ispp, a_dtype);
+  if (small_mxfp4_ok(a_dtype, M, top_k, E, hidden, ispp, A, w13, w13_scale, w2, w2_scale))
+    return launch_small_mxfp4(static_cast<const uint16_t*>(A), M, hidden, w13, w13_scale, w2, w2_scale, E, ispp,
+                              b13, b2, swiglu_limit, topk_ids, mul_routed_weight ? topk_w : nullptr, top_k,
+                              expert_map, num_global_experts, at<uint16_t>(workspace, plan.act),
+                              static_cast<uint16_t*>(out), stream);
   if (!plan.stream && !mxfp4_tile_fits(M, top_k, hidden, ispp)) {
     // a batch whose activations reach 2^31 bytes runs as consecutive token
     // chunks (a token's output depends only on its own slots); each lays out
