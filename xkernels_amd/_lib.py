@@ -104,11 +104,11 @@ def last_error() -> str:
 
 def call(name: str, *args) -> None:
     """Invoke an entry point that returns a status; raise on failure."""
-    rc = getattr(load(), name)(*args)
+    rc = getattr(_LIB or load(), name)(*args)
     if rc != XK_OK:
         raise RuntimeError(f"{name} failed (status {rc}): {last_error()}")
 
 
 def query(name: str, *args) -> int:
     """Invoke a size query (no status)."""
-    return int(getattr(load(), name)(*args))
+    return getattr(_LIB or load(), name)(*args)

@@ -23,31 +23,38 @@ _ROUTER_DT = {**_DT, torch.float16: _lib.XK_DT_FP16}
 
 
 def _need_gpu(op: str, *tensors: torch.Tensor | None) -> torch.device:
-    dev = None
+    first = None
     for t in tensors:
         if t is None:
             continue
         if not t.is_cuda:
             raise RuntimeError(f"{op}: the HIP backend needs device tensors, got {t.device}")
-        if dev is None:
-            dev = t.device
-        elif t.device != dev:
-            raise RuntimeError(f"{op}: tensors on different devices ({dev} vs {t.device})")
-    return dev
+        if first is None:
+            first = t
+        elif t.get_device() != first.get_device():
+            raise RuntimeError(f"{op}: tensors on different devices ({first.device} vs {t.device})")
+    return first.device
 
 
 def _ptr(t: torch.Tensor | None) -> int | None:
     return None if t is None else t.data_ptr()
 
 
+# the current stream's handle without building a Stream object (about 1 us a
+# call), where this torch has the call
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream(dev: torch.device) -> int:
+    if _raw_stream is not None:
+        return _raw_stream(dev.index)
     return torch.cuda.current_stream(dev).cuda_stream
 
 
 def _contig(t: torch.Tensor, dtype: torch.dtype | None = None) -> torch.Tensor:
     if dtype is not None and t.dtype != dtype:
         t = t.to(dtype)
-    return t.contiguous()
+    return t if t.is_contiguous() else t.contiguous()
 
 
 def _dtype_code(op: str, t: torch.Tensor) -> int:
@@ -158,11 +165,11 @@ def moe_int4_w4a16_hip(A: torch.Tensor, packed: torch.Tensor, scale: torch.Tenso
     ids = _contig(topk_ids, torch.int32)
     tw = _contig(topk_w, torch.float32)
     emap, n_global = _emap(expert_map, dev)
-    nbytes = _lib.query("xk_moe_int4_w4a16_ep_workspace_bytes", M, top_k, E, N, K, n_global)
     if isinstance(workspace, MoeInt4Workspace) and workspace.matches(M, top_k, N, dtype=A.dtype, device=dev):
         out = workspace.out[:M]
         scratch = workspace.scratch_for(M, E, N, K, num_global_experts=n_global)
     else:
+        nbytes = _lib.query("xk_moe_int4_w4a16_ep_workspace_bytes", M, top_k, E, N, K, n_global)
         out = torch.empty((M, N), dtype=A.dtype, device=dev)
         scratch = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=dev)
     _lib.call(
@@ -190,20 +197,14 @@ def moe_mxfp4_hip(A: torch.Tensor, w13: torch.Tensor, w13_scale: torch.Tensor, w
     top_k = topk_ids.shape[1]
     if group_size != 32:
         raise RuntimeError(f"moe_mxfp4: group_size={group_size}; MXFP4 blocks are 32 elements")
-    checks = {
-        "w13": (tuple(w13.shape), (E, 2 * ispp, hidden // 2)),
-        "w13_scale": (tuple(w13_scale.shape), (E, 2 * ispp, hidden // 32)),
-        "w2": (tuple(w2.shape), (E, hidden, ispp // 2)),
-        "w2_scale": (tuple(w2_scale.shape), (E, hidden, ispp // 32)),
-        "topk_w": (tuple(topk_w.shape), (M, top_k)),
-    }
-    if b13 is not None:
-        checks["b13"] = (tuple(b13.shape), (E, 2 * ispp))
-    if b2 is not None:
-        checks["b2"] = (tuple(b2.shape), (E, hidden))
-    for name, (got, want) in checks.items():
-        if got != want:
-            raise RuntimeError(f"moe_mxfp4: {name} shape {got} != {want}")
+    for name, t, want in (("w13", w13, (E, 2 * ispp, hidden // 2)),
+                          ("w13_scale", w13_scale, (E, 2 * ispp, hidden // 32)),
+                          ("w2", w2, (E, hidden, ispp // 2)),
+                          ("w2_scale", w2_scale, (E, hidden, ispp // 32)),
+                          ("topk_w", topk_w, (M, top_k)),
+                          ("b13", b13, (E, 2 * ispp)), ("b2", b2, (E, hidden))):
+        if t is not None and t.shape != want:
+            raise RuntimeError(f"moe_mxfp4: {name} shape {tuple(t.shape)} != {want}")
     if w13.dtype != torch.uint8 or w2.dtype != torch.uint8:
         raise RuntimeError("moe_mxfp4: packed weights must be uint8")
     a_dt = _dtype_code("moe_mxfp4", A)
