@@ -137,3 +137,15 @@ def test_auto_dispatch_above_2048_experts(dev):
     assert torch.equal(ids.cpu(), rids)
     torch.testing.assert_close(w.cpu(), rw, rtol=1e-5, atol=1e-6, equal_nan=True)
     assert ids[1].tolist() == list(range(6))
+
+
+@pytest.mark.parametrize("M,E,k", [(1, 1, 1), (15, 127, 16), (17, 128, 8), (16, 129, 1), (33, 255, 16), (5, 256, 16),
+                                   (31, 257, 9), (18, 384, 6), (7, 505, 16), (9, 512, 16), (9, 512, 17), (9, 513, 16)])
+@pytest.mark.parametrize("dt", DTYPES)
+def test_16_lane_rows_edges(M, E, k, dt, dev):
+    """Around the limits of the 16-lane rows (512 experts, k = 16), their
+    register sizes (128, 256) and their wide loads (E % 8, row alignment)."""
+    g = torch.randn(M + 1, E, generator=torch.Generator(device=dev).manual_seed(E * k), device=dev).to(dt)
+    for rows in (g[:M], g[1:]):  # the second starts at another alignment for odd E
+        _check(rows, k, True)
+        _check(rows, k, False)
