@@ -370,38 +370,68 @@ __device__ __forceinline__ void run_tile(const TileArgs& p, int e, int col_tile,
     });
 
   // C layout: register v of a lane is row 8 (v / 4) + 4 h + v % 4, column c32.
+  auto slot_of = [&](int i, int v) { return slot_lds[32 * i + 8 * (v >> 2) + 4 * h + (v & 3)]; };
+  if constexpr (EPI == Epi::kRows) {
 #pragma unroll
-  for (int i = 0; i < RT; ++i)
+    for (int i = 0; i < RT; ++i)
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const int slot = slot_lds[32 * i + 8 * (v >> 2) + 4 * h + (v & 3)];
-      if constexpr (EPI == Epi::kRows) {
+      for (int v = 0; v < 16; ++v) {
+        const int slot = slot_of(i, v);
         float* orow = static_cast<float*>(p.out) + static_cast<int64_t>(slot) * ncols;
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
           const int col = col0 + 32 * t + c32;
           if (slot >= 0 && col < ncols) orow[col] = acc[i][t][v];
         }
-      } else if constexpr (EPI == Epi::kGateUp) {
-        const int col = col0 + c32;
-        if (slot >= 0 && col < ncols) {
-          const uint16_t* b = p.bias ? p.bias + static_cast<int64_t>(e) * p.N : nullptr;
-          static_cast<uint16_t*>(p.out)[static_cast<int64_t>(slot) * ncols + col] =
-              mxfp4_swiglu(acc[i][0][v], acc[i][1][v], b, col, ncols, p.limit);
-        }
-      } else {
-        uint16_t* orow = static_cast<uint16_t*>(p.out) + static_cast<int64_t>(slot) * ncols;
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-          const int col = col0 + 32 * t + c32;
-          if (slot >= 0 && col < ncols) {
-            float d = round_bf16(acc[i][t][v]);
-            if (p.bias != nullptr) d = d + bf16_to_f32(p.bias[static_cast<int64_t>(e) * ncols + col]);
-            orow[col] = f32_to_bf16(d);
-          }
-        }
       }
-    }
+    return;
+  }
+  // bf16 outputs leave two columns at a time: a lane pair (c, c + 1) holds two
+  // bf16 each in a register, of column tiles 0 and 1 (kDown) or of rows v and
+  // v + 1 (kGateUp); the even lane takes both low halves, the odd lane both
+  // high ones. The columns are multiples of 32 wide, so a tile is in or out.
+  const bool odd = (lane & 1) != 0;
+  const uint32_t pair_sel = odd ? 0x03020706u : 0x05040100u;
+  auto pair_up = [&](uint32_t x) __attribute__((always_inline)) {
+    const uint32_t y = __builtin_amdgcn_update_dpp(x, x, 0xB1, 0xF, 0xF, false);  // the neighbour's
+    return __builtin_amdgcn_perm(y, x, pair_sel);
+  };
+  uint16_t* const out16 = static_cast<uint16_t*>(p.out);
+  if constexpr (EPI == Epi::kGateUp) {
+    const int col = col0 + (c32 & ~1);
+    if (col0 >= ncols) return;
+    const uint16_t* b = p.bias ? p.bias + static_cast<int64_t>(e) * p.N : nullptr;
+#pragma unroll
+    for (int i = 0; i < RT; ++i)
+#pragma unroll
+      for (int v = 0; v < 16; v += 2) {
+        uint32_t x = mxfp4_swiglu(acc[i][0][v], acc[i][1][v], b, col0 + c32, ncols, p.limit);
+        x |= static_cast<uint32_t>(mxfp4_swiglu(acc[i][0][v + 1], acc[i][1][v + 1], b, col0 + c32, ncols, p.limit)) << 16;
+        const uint32_t o = pair_up(x);
+        const int slot = slot_of(i, v + (odd ? 1 : 0));
+        if (slot >= 0) *reinterpret_cast<uint32_t*>(out16 + static_cast<int64_t>(slot) * ncols + col) = o;
+      }
+  } else {
+    const int col = col0 + (odd ? 32 : 0) + (c32 & ~1);
+    float b[2] = {0.f, 0.f};
+    if (p.bias != nullptr)
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+        b[t] = bf16_to_f32(p.bias[static_cast<int64_t>(e) * ncols + min(col0 + 32 * t + c32, ncols - 1)]);
+#pragma unroll
+    for (int i = 0; i < RT; ++i)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        float d[2] = {acc[i][0][v], acc[i][1][v]};
+        if (p.bias != nullptr)
+#pragma unroll
+          for (int t = 0; t < 2; ++t) d[t] = round_bf16(d[t]) + b[t];
+        const uint32_t o = pair_up(f32_to_bf16(d[0]) | static_cast<uint32_t>(f32_to_bf16(d[1])) << 16);
+        const int slot = slot_of(i, v);
+        if (slot >= 0 && col < ncols)
+          *reinterpret_cast<uint32_t*>(out16 + static_cast<int64_t>(slot) * ncols + col) = o;
+      }
+  }
 }
 
 template <Fmt FMT, bool SCL, Epi EPI, int MAXRT>
