@@ -270,3 +270,17 @@ def test_topk_softmax_rejects_bad_arguments(kw):
 
 def test_topk_softmax_empty_batch_is_ok():
     assert _rc("xk_moe_topk_softmax", None, 0, 0, 64, 8, 1, None, None, None) == _lib.XK_OK
+
+
+def test_stage_entry_keeps_padded_shapes_on_the_stream_kernel():
+    """K or N not a multiple of 256 and many rows per expert: the fused call takes
+    the tile kernel, the stage entry the stream kernel, whose plane count it
+    answers and whose calls may come without align outputs."""
+    q = lambda name, *a: _lib.query(name, *a)
+    for N, K in ((2880, 2880), (4096, 7200), (48, 2048)):
+        assert q("xk_moe_int4_kernel", 600, 4, 48, N, K, _lib.XK_DT_BF16, 32, 0, 0) == 2
+        parts = q("xk_moe_int4_gemm_parts", 600, 4, 48, N, K, _lib.XK_DT_BF16, 32, 0)
+        assert parts == q("xk_moe_int4_gemm_parts", 600, 4, 48, N, K, _lib.XK_DT_BF16, 32,
+                          _lib._XK_INT4_TEST_FORCE_STREAM)
+    assert _rc("xk_moe_int4_w4a16_gemm", FAKE, 0, 4, 64, FAKE, FAKE, 2, 16, 32, FAKE, 2, None, 0, FAKE, FAKE,
+               FAKE, 1 << 10, None, 0, None) == _lib.XK_ERR_INVALID  # internal, not a caller's

@@ -144,8 +144,9 @@ using namespace xk;
 namespace xk {
 namespace {
 constexpr int64_t kNoAllocScratchBytes = int64_t(64) << 20;
+constexpr int64_t kNoAllocExtra = int64_t(64) << 10;  // the align's grid scratch, not counted in the limit
 constexpr int kMaxDevices = 64;
-static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
+static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes + kNoAllocExtra];
 std::mutex g_scratch_mu;
 void* g_scratch_dev[kMaxDevices] = {};
 
@@ -206,7 +207,7 @@ int32_t xk_moe_int4_block_size(int64_t M, int64_t top_k, int64_t E) {
 int32_t xk_moe_int4_kernel(int64_t M, int64_t top_k, int64_t E, int64_t N, int64_t K,
                            int32_t a_dtype, int32_t group_size, int32_t flags,
                            int32_t num_global_experts) {
-  return int4_kernel_code(M, top_k, E, N, K, a_dtype, group_size, flags,
+  return int4_kernel_code(M, top_k, E, N, K, a_dtype, group_size, flags | XK_INT4_FUSED,
                           num_global_experts > E ? num_global_experts : 0);
 }
 
@@ -224,11 +225,13 @@ namespace {
 // under an expert map of ep_global > E experts, the expert-parallel choice's.
 int64_t int4_fused_planes(int64_t M, int64_t top_k, int64_t E, int64_t N, int64_t K,
                           int64_t ep_global) {
-  int64_t p = std::max(int4_gemm_parts(M, top_k, E, N, K, XK_DT_BF16, 32, 0),
-                       int4_gemm_parts(M, top_k, E, N, K, XK_DT_FP32, 32, 0));
-  if (ep_global > E)
-    p = std::max<int64_t>(p, std::max(int4_gemm_parts(M, top_k, E, N, K, XK_DT_BF16, 32, 0, ep_global),
-                                      int4_gemm_parts(M, top_k, E, N, K, XK_DT_FP32, 32, 0, ep_global)));
+  // (0 slices more than XK_INT4_FUSED for padded shapes: those the stage entry's
+  // choice would write)
+  int64_t p = 1;
+  for (const int flags : {0, XK_INT4_FUSED})
+    for (const int dt : {XK_DT_BF16, XK_DT_FP32})
+      for (const int64_t ep : {int64_t(0), ep_global > E ? ep_global : 0})
+        p = std::max<int64_t>(p, int4_gemm_parts(M, top_k, E, N, K, dt, 32, flags, ep));
   return p;
 }
 int64_t int4_planes_offset(int64_t M, int64_t top_k, int64_t E, int64_t K) {
@@ -266,6 +269,8 @@ int xk_moe_int4_w4a16_gemm(const void* A, int32_t a_dtype, int64_t M, int64_t K,
                            float* slot_out, int32_t flags, void* workspace,
                            int64_t workspace_bytes, hipStream_t stream) {
   clear_error();
+  XK_REQUIRE((flags & ~(XK_INT4_TEST_FORCE_TILE | XK_INT4_TEST_FORCE_STREAM)) == 0,
+             "int4: unknown flags 0x%x (pass 0)", flags);
   return launch_int4_gemm(A, a_dtype, M, K, packed, scale, E, N, group_size, topk_ids, top_k,
                           expert_map, num_global_experts, sorted_token_ids, expert_offsets,
                           slot_out, flags, 0, workspace, workspace_bytes, false, stream);
@@ -313,10 +318,11 @@ int xk_moe_int4_w4a16(const void* A, int32_t a_dtype, int64_t M, int64_t K,
   // order), so the chunks write what one call would, bit for bit, with the
   // MFMA kernels instead of the scalar one. Each chunk lays out its smaller
   // workspace at the start of this one; the stream orders them.
-  if (flags == 0 && int4_kernel_code(M, top_k, E, N, K, a_dtype, group_size, 0, 0) == 0) {
+  const int fused = flags | XK_INT4_FUSED;
+  if (flags == 0 && int4_kernel_code(M, top_k, E, N, K, a_dtype, group_size, fused, 0) == 0) {
     const int64_t elem = a_dtype == XK_DT_FP32 ? 4 : 2;
     int64_t mc = ((int64_t(1) << 31) - 1) / (K * elem);
-    while (mc > 0 && int4_kernel_code(mc, top_k, E, N, K, a_dtype, group_size, 0, 0) == 0) mc /= 2;
+    while (mc > 0 && int4_kernel_code(mc, top_k, E, N, K, a_dtype, group_size, fused, 0) == 0) mc /= 2;
     if (mc > 0 && mc < M) {
       mc = cdiv(M, cdiv(M, mc));  // even parts: a short last one would take another kernel's summation order
       for (int64_t m0 = 0; m0 < M; m0 += mc) {
@@ -343,9 +349,9 @@ int xk_moe_int4_w4a16(const void* A, int32_t a_dtype, int64_t M, int64_t K,
   // sizes for it); else, and with the test bits, every slot counts.
   int64_t ep_global = 0;
   if (flags == 0 && expert_map != nullptr && num_global_experts > E &&
-      int4_gemm_parts(M, top_k, E, N, K, a_dtype, group_size, 0, num_global_experts) <= planes_held)
+      int4_gemm_parts(M, top_k, E, N, K, a_dtype, group_size, fused, num_global_experts) <= planes_held)
     ep_global = num_global_experts;
-  const int64_t parts = int4_gemm_parts(M, top_k, E, N, K, a_dtype, group_size, flags, ep_global);
+  const int64_t parts = int4_gemm_parts(M, top_k, E, N, K, a_dtype, group_size, fused, ep_global);
   // the test bits may force a kernel that writes more partial planes than the
   // default choices the workspace is sized for
   XK_REQUIRE(parts <= planes_held,
@@ -355,7 +361,7 @@ int xk_moe_int4_w4a16(const void* A, int32_t a_dtype, int64_t M, int64_t K,
   const int32_t* offsets = nullptr;
   // the decode kernel routes for itself; the other MFMA kernels take the align
   if (int4_use_stream(a_dtype, group_size, K) &&
-      !int4_gemm_self_routes(M, top_k, E, N, K, a_dtype, group_size, flags, ep_global)) {
+      !int4_gemm_self_routes(M, top_k, E, N, K, a_dtype, group_size, fused, ep_global)) {
     int rc = launch_align(topk_ids, numel, int(E), int4_block_size(), expert_map,
                           num_global_experts, at<int32_t>(workspace, al.sorted),
                           at<int32_t>(workspace, al.expert_ids),
@@ -369,7 +375,7 @@ int xk_moe_int4_w4a16(const void* A, int32_t a_dtype, int64_t M, int64_t K,
   }
   if (int rc = launch_int4_gemm(A, a_dtype, M, K, packed, scale, E, N, group_size, topk_ids,
                                 top_k, expert_map, num_global_experts, sorted, offsets,
-                                slot_out, flags, ep_global, at<char>(workspace, al.total),
+                                slot_out, fused, ep_global, at<char>(workspace, al.total),
                                 round_up(int4_gemm_workspace_bytes(M, K)), sorted != nullptr, stream))
     return rc;
   return launch_topk_combine(slot_out, M, top_k, N, topk_w, mul_routed_weight, topk_ids,
@@ -394,7 +400,10 @@ int xk_moe_int4_w4a16_noalloc(const void* A, int32_t a_dtype, int64_t M, int64_t
              "int4 noalloc: unknown flags 0x%x (pass 0)", flags);
   if (M == 0) return XK_OK;
   const int64_t need = xk_moe_int4_w4a16_workspace_bytes(M, top_k, E, N, K);
-  XK_REQUIRE(need <= xk::kNoAllocScratchBytes,
+  // the grid align's scratch of a batch one workgroup could sort does not count
+  const int64_t grid = M * top_k <= 8192 && E <= 512 ? round_up(align_workspace_bytes(M * top_k, int(E))) : 0;
+  static_assert(8 * 512 * 4 <= xk::kNoAllocExtra, "8192 slots' histograms fit the extra bytes");
+  XK_REQUIRE(need - grid <= xk::kNoAllocScratchBytes,
              "int4 noalloc: the call needs %lld B of scratch, above the fixed %lld B "
              "(use xk_moe_int4_w4a16 with a workspace)",
              (long long)need, (long long)xk::kNoAllocScratchBytes);
@@ -402,7 +411,7 @@ int xk_moe_int4_w4a16_noalloc(const void* A, int32_t a_dtype, int64_t M, int64_t
   if (int rc = xk::noalloc_scratch(&ws)) return rc;
   return xk_moe_int4_w4a16(A, a_dtype, M, K, packed, scale, E, N, group_size, topk_ids, topk_w,
                            top_k, expert_map, num_global_experts, mul_routed_weight, flags, out,
-                           ws, xk::kNoAllocScratchBytes, stream);
+                           ws, xk::kNoAllocScratchBytes + xk::kNoAllocExtra, stream);
 }
 
 int xk_moe_topk_softmax(const void* gating_output, int32_t dtype, int64_t M, int64_t E,

@@ -8,3 +8,8 @@
 
 #define XK_INT4_TEST_FORCE_TILE (1 << 8)
 #define XK_INT4_TEST_FORCE_STREAM (1 << 9)
+// Set by the fused call (and the query of its kernel) alone, never accepted from
+// a caller: K or N not a multiple of 256 may take the tile kernel. The stage
+// entry keeps such shapes on the stream kernel, whose calls may come without
+// align outputs and with the plane count it answers.
+#define XK_INT4_FUSED (1 << 10)
