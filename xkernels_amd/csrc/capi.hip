@@ -437,7 +437,7 @@ int xk_moe_topk_softmax(const void* gating_output, int32_t dtype, int64_t M, int
 namespace {
 
 // The MXFP4 pipeline: both projections through the stream kernel (bf16
-// activations, few routed rows per expert, shapes within its limits), else
+// activations, few routed rows per expert, sizes multiples of 64), else
 // through the tile kernel.
 // Workspace after the align scratch: act [numel, ispp] bf16, then the stream
 // path's down planes [S1, numel, hidden] fp32 and gate/up planes [S0, numel,
@@ -458,10 +458,11 @@ struct Mxfp4Plan {
   bool stream;
   int s0, s1;
   int64_t act, down, gu, abf, queue, total;
-  Mxfp4Plan(int64_t M, int64_t top_k, int64_t E, int64_t hidden, int64_t ispp, int a_dtype) {
+  Mxfp4Plan(int64_t M, int64_t top_k, int64_t E, int64_t hidden, int64_t ispp, int a_dtype,
+            bool tile_only = false) {
     const int64_t numel = M * top_k;
     AlignScratch al(numel, int(E), mxfp4_block_size());
-    stream = a_dtype == XK_DT_BF16 && numel > 0 && numel < kMxStreamRowsPerExpert * E &&
+    stream = !tile_only && a_dtype == XK_DT_BF16 && numel > 0 && numel < kMxStreamRowsPerExpert * E &&
              mxfp4_rs_ok(M, hidden, 2 * ispp, E, numel) &&
              mxfp4_rs_ok(numel, ispp, hidden, E, numel);
     s0 = stream ? mxfp4_rs_slices(hidden, 2 * ispp, numel, E) : 0;
@@ -518,7 +519,14 @@ int xk_moe_mxfp4(const void* A, int32_t a_dtype, int64_t M, int64_t hidden, cons
   if (workspace == nullptr || workspace_bytes < need)
     return set_error(XK_ERR_WORKSPACE, "mxfp4: workspace %lld B < %lld B",
                      (long long)workspace_bytes, (long long)need);
-  const Mxfp4Plan plan(M, top_k, E, hidden, ispp, a_dtype);
+  // sizes that are not multiples of 128: 16-byte aligned pointers are required,
+  // and the stream kernel reads scales two bytes at a time
+  const bool odd = hidden % 128 != 0 || ispp % 128 != 0;
+  auto low_bits = [](const void* x) { return reinterpret_cast<uintptr_t>(x); };
+  XK_REQUIRE(!odd || (low_bits(A) | low_bits(w13) | low_bits(w2)) % 16 == 0,
+             "mxfp4: activations and weights must be 16-byte aligned");
+  const Mxfp4Plan plan(M, top_k, E, hidden, ispp, a_dtype,
+                       odd && (low_bits(w13_scale) | low_bits(w2_scale)) % 2 != 0);
   if (small_mxfp4_ok(a_dtype, M, top_k, E, hidden, ispp, A, w13, w13_scale, w2, w2_scale))
     return launch_small_mxfp4(static_cast<const uint16_t*>(A), M, hidden, w13, w13_scale, w2, w2_scale, E, ispp,
                               b13, b2, swiglu_limit, topk_ids, mul_routed_weight ? topk_w : nullptr, top_k,

@@ -778,6 +778,14 @@ mxfp4_stream_rs_padk(RsArgs p) {
   stream_body<kFmtFp4, 4>(p);
 }
 
+// An even number of scales per row that is not a multiple of four (K a multiple
+// of 64): 2-byte scale loads.
+__global__ void __launch_bounds__(kRsThreads)
+__attribute__((amdgpu_waves_per_eu(kRsWaves / 4, kRsWaves / 4)))
+mxfp4_stream_rs_sld2(RsArgs p) {
+  stream_body<kFmtFp4, 2>(p);
+}
+
 }  // namespace
 
 // K slices for one 16-row pass: the fewest (the ceil(K / 256) lines split
@@ -855,7 +863,7 @@ int launch_int4_rs(const void* A, bool f32a, int64_t M, int64_t K, const int32_t
 }
 
 bool mxfp4_rs_ok(int64_t a_rows, int64_t K, int64_t N, int64_t E, int64_t numel) {
-  const int s = K % 128 == 0 ? mxfp4_rs_slices(K, N, numel, E) : 0;  // 4-byte scale rows
+  const int s = K % 64 == 0 ? mxfp4_rs_slices(K, N, numel, E) : 0;  // 2-byte scale rows
   return s > 0 && N % 32 == 0 && E <= kRsMaxE && N * (K / 2) < (int64_t(1) << 31) &&
          a_rows * K * 2 < (int64_t(1) << 31) && numel * N * 4 * s < (int64_t(1) << 31);
 }
@@ -867,12 +875,8 @@ int launch_mxfp4_rs(const void* A, int64_t a_rows, int64_t K, const uint8_t* w, 
   RsArgs a{static_cast<const uint16_t*>(A), reinterpret_cast<const uint32_t*>(w), ws, sorted_ids,
            offsets, topk_ids, emap, num_global, planes, int(K), int(N), int(E), int(numel), 1,
            int(a_row_div), mxfp4_rs_slices(K, N, numel, E), static_cast<uint32_t>(a_rows * K * 2), 0};
-  if (K % 256 == 0)
-    hipLaunchKernelGGL(mxfp4_stream_rs, dim3(static_cast<unsigned>(device_cu_count())),
-                       dim3(kRsThreads), 0, stream, a);
-  else
-    hipLaunchKernelGGL(mxfp4_stream_rs_padk, dim3(static_cast<unsigned>(device_cu_count())),
-                       dim3(kRsThreads), 0, stream, a);
+  hipLaunchKernelGGL(K % 256 == 0 ? mxfp4_stream_rs : K % 128 == 0 ? mxfp4_stream_rs_padk : mxfp4_stream_rs_sld2,
+                     dim3(static_cast<unsigned>(device_cu_count())), dim3(kRsThreads), 0, stream, a);
   XK_CHECK_LAUNCH("mxfp4_stream_rs");
   return XK_OK;
 }
