@@ -35,10 +35,41 @@ def test_int4_tile_edges(N, K, gs, dev):
     ids = _row_ids(ROWS, K)
     print(f"int4 tile N={N} K={K} gs={gs}", flush=True)
     A, packed, scale, ids = _device_inputs(ids.shape[0], len(ROWS), N, K, ids, seed=K + N, gs=gs)
-    # 72 rows per expert on average: the 128-row kernel
+    # 77 rows per expert on average: the 128-row kernel
     rows = _gemm_rows(A, packed, scale, ids, flags=_lib._XK_INT4_TEST_FORCE_TILE, gs=gs)
     assert not torch.isnan(rows).any(), "a routed slot's row was not written"
     _bounded_check(A, packed, scale, ids, rows, gs=gs)
+
+
+@pytest.mark.parametrize("N", [16, 48, 272])
+@pytest.mark.parametrize("K,gs", [(32, 32), (160, 32), (2080, 32), (192, 64), (2048, 32)])
+@pytest.mark.parametrize("M", [1, 2])
+def test_int4_tile_of_one_row(N, K, gs, M, dev):
+    """Activations, weights and scales that are shorter than the last chunk's
+    offset into them: the loads past K, past N and of pad rows return zeros
+    whatever part of their offset the range check counts."""
+    print(f"int4 tile M={M} N={N} K={K} gs={gs}", flush=True)
+    ids = torch.tensor([[1], [0]][:M], dtype=torch.int32)
+    A, packed, scale, ids = _device_inputs(M, 2, N, K, ids, seed=K + N + M, gs=gs)
+    rows = _gemm_rows(A, packed, scale, ids, flags=_lib._XK_INT4_TEST_FORCE_TILE, gs=gs)
+    assert not torch.isnan(rows).any(), "a routed slot's row was not written"
+    _bounded_check(A, packed, scale, ids, rows, gs=gs)
+
+
+@pytest.mark.parametrize("hidden,ispp", [(32, 32), (32, 160), (160, 32), (2080, 160), (160, 2080)])
+def test_mxfp4_one_token(hidden, ispp, dev):
+    """The same for one token's activation row in both MXFP4 projections."""
+    print(f"mxfp4 one token hidden={hidden} ispp={ispp}", flush=True)
+    wts = make_mxfp4_moe_weights(2, hidden, ispp, with_bias=True, device="cpu", seed=ispp, scale_lo=115, scale_hi=122)
+    A = torch.randn(1, hidden, generator=torch.Generator().manual_seed(3)).to(torch.bfloat16)
+    ids, w = torch.tensor([[1]], dtype=torch.int32), torch.full((1, 1), 0.7)
+    keys = ("w13", "w13_scale", "w2", "w2_scale")
+    got = fused_moe_mxfp4(A.to(dev), *(wts[k].to(dev) for k in keys), ids.to(dev), w.to(dev),
+                          b13=wts["b13"].to(dev), b2=wts["b2"].to(dev), backend=Backend.HIP).float().cpu()
+    want = moe_mxfp4_ref(A, *(wts[k] for k in keys), ids, w, b13=wts["b13"], b2=wts["b2"]).float()
+    # one slot of few columns: a bf16 rounding of a sum that falls on the other
+    # side of a tie moves that column by 2^-8 of its size
+    assert float((got - want).norm() / want.norm()) < 4e-3
 
 
 @pytest.mark.parametrize("hidden,ispp", [(512, 512), (1024, 160), (96, 512), (32, 32), (2080, 96), (544, 1536)])

@@ -137,8 +137,10 @@ __device__ __forceinline__ void run_tile(const TileArgs& p, int e, int col_tile,
     const int col = EPI == Epi::kGateUp ? col0 : col0 + 32 * t;
     const int valid = max(0, min(32, ncols - col));
     const int64_t row = static_cast<int64_t>(e) * p.N + min(col, ncols - 1) + (EPI == Epi::kGateUp ? t * ncols : 0);
-    rw[t] = uniform_rsrc(p.w + row * KB, valid * KB);
-    rs[t] = uniform_rsrc(p.scale + row * G * SB, valid * G * SB);
+    // a tile past the last column keeps one row (of it the last one; never
+    // stored): an empty buffer would be smaller than the scalar offsets
+    rw[t] = uniform_rsrc(p.w + row * KB, max(valid, 1) * KB);
+    rs[t] = uniform_rsrc(p.scale + row * G * SB, max(valid, 1) * G * SB);
   }
   const i32x4 ra = make_rsrc(p.A, p.a_bytes);
   constexpr int kOut = static_cast<int>(0x80000000u);  // past every buffer
@@ -158,9 +160,10 @@ __device__ __forceinline__ void run_tile(const TileArgs& p, int e, int col_tile,
     for (int g = 0; g < 2; ++g) {
       const int k0 = ch * kChunkK + g * kStageK;
       const bool past = SCL && k0 + a_piece * 8 >= K;
+      const int soff = !SCL || k0 < K ? k0 * 2 : 0;
 #pragma unroll
       for (int i = 0; i < RT; ++i)
-        dma_16(ra, a_lds + ((buf * 2 + g) * RT + i) * 256 + wave * 64, past ? kOut : a_off[i], k0 * 2);
+        dma_16(ra, a_lds + ((buf * 2 + g) * RT + i) * 256 + wave * 64, past ? kOut : a_off[i], soff);
     }
   };
 
@@ -174,9 +177,11 @@ __device__ __forceinline__ void run_tile(const TileArgs& p, int e, int col_tile,
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
 #pragma unroll
-      for (int g = 0; g < 2; ++g)
+      for (int g = 0; g < 2; ++g) {
+        const bool past = SCL && 4 * ch + 2 * g + h >= (K >> 5);
         k.w[g][t] = __builtin_bit_cast(
-            u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw[t], w_off + 32 * g, ch * 64, 0));
+            u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw[t], past ? kOut : w_off + 32 * g, ch * 64, 0));
+      }
       if constexpr (SCL) {
 #pragma unroll
         for (int g = 0; g < 2; ++g) {
