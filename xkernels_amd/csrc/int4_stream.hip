@@ -81,6 +81,7 @@ template <int FMT> struct RsFmt {
 };
 constexpr int kRsRing = 2;                    // ring slots: lines k+1 .. k+R-1 in flight while line k computes
 constexpr int kRsLdsA = 112 * 1024;         // bytes of LDS for one activation slice
+constexpr int kRsPast = static_cast<int>(0x80000000u);  // a load offset past every buffer: lands zeros
 constexpr int kRsMaxE = 512;
 constexpr int kRsMaxSelf = 4096;            // routed slots a workgroup can route for itself
 
@@ -129,9 +130,13 @@ __device__ __forceinline__ f32x4 quad_transpose(f32x4 e) {
 // SLD: bytes per block-start scale load. 16 when K is a multiple of 256 and
 // every scale row a 16-byte multiple; else (PADK) 4-byte loads, or 2-byte ones
 // for an odd number of scales per row: each lies wholly inside or wholly past
-// the buffer (a 16-byte load that straddles the end of the scales comes back
+// the row (a 16-byte load that straddles the end of the scales comes back
 // empty, real bytes included) and needs only 4- (2-) byte aligned rows. K not
-// a multiple of 256 zero-pads the last line's activations.
+// a multiple of 256: activations and scales past K are zero. The weights there
+// are another column's (or zero past the buffer), and with that column's scales
+// they would put a NaN into this one where they decode to an infinity (e8m0
+// bytes 253 and 254, an infinite bf16 scale). Scalar offsets stay below the
+// buffer's size, so that the range check's difference of the two never wraps.
 // F32A (INT4 only): fp32 activations, whose reference contraction uses the
 // exact products (n - 8) s. The activations are staged as a bf16 pair hi + lo
 // (A - hi - lo <= 2^-16 |A|), the weights split exactly (dequant_split_nat),
@@ -373,27 +378,15 @@ __device__ __forceinline__ void stream_body(const RsArgs& p) {
     }
     // rows of pad slots read nothing (an offset past A; their LDS rows only
     // feed output rows that are never stored)
-    const int a_voff = sid >= 0 ? (sid / p.a_row_div) * K * 2 + q * 64 : (1 << 30);
+    const int a_voff = sid >= 0 ? (sid / p.a_row_div) * K * 2 + q * 64 : kRsPast;
     for (int blk = wave; blk < nblk; blk += kRsWaves) {
       const int j = blk & 3, h = (blk >> 2) & 1, line = blk >> 3;
-      dma_16(ra, &a_lds[blk * 64], a_voff, (s * Ks + line * 256 + 128 * h + 8 * j) * 2);
+      const int k0 = s * Ks + line * 256 + 128 * h + 8 * j;  // of lanes q = 0
+      dma_16(ra, &a_lds[blk * 64], PADK && 32 * q >= K - k0 ? kRsPast : a_voff, !PADK || k0 < K ? k0 * 2 : 0);
     }
     if (first) count_steps();  // while the loads are in flight
     XK_WAIT_VMCNT(0);
     lds_sync();
-    if constexpr (PADK) {
-      if (s * Ks + Ks > K) {
-        // the slice runs past K: its activations there are zero (the weights
-        // and scales the stream reads there are finite: other columns' data,
-        // or zero past the buffer), after every wave's loads have landed
-        for (int t = tid; t < nblk * 64; t += kRsThreads) {
-          const int blk = t >> 6, qq = (t & 63) >> 4;
-          const int j = blk & 3, h = (blk >> 2) & 1, line = blk >> 3;
-          if (s * Ks + line * 256 + (4 * h + qq) * 32 + 8 * j >= K) a_lds[t] = u32x4{0u, 0u, 0u, 0u};
-        }
-        lds_sync();
-      }
-    }
   };
 
   // One chunk: this wave's `cnt` column pairs from `my_lo` of expert e,
@@ -468,30 +461,32 @@ __device__ __forceinline__ void stream_body(const RsArgs& p) {
       // per column)
       const bool blk = uniform(((pl & (kRsScLines - 1)) == 0 && pst < steps) ? 1 : 0) != 0;
       const int lines_left = nl - pl;  // scalar: the per-lane test below is one compare
+      // a half pair's second tile lies past N (N % 32 is 0 for MXFP4) and loads
+      // the first one's rows
+      const int tile = PADK && FMT == kFmtInt4 && cp * 32 + 16 >= N ? 0 : 16;
 #pragma unroll
       for (int c = 0; c < 2; ++c) {
 #pragma unroll
         for (int h = 0; h < 2; ++h)
-          sl.w[c][h] = __builtin_amdgcn_raw_buffer_load_b128(rw, w_lane + 64 * h, wo + c * 16 * KW * 4,
-                                                             0);
+          sl.w[c][h] = __builtin_amdgcn_raw_buffer_load_b128(rw, w_lane + 64 * h, wo + c * tile * KW * 4, 0);
         if (blk) {  // lanes past the slice's last line read nothing (offset past the buffer)
 #pragma unroll
           for (int i = 0; i < F::kScLoads; ++i)
           {
             const int lines = F::kLinesPerLoad << glog;  // lines one 16-byte piece covers
             const bool in = (q + 4 * i) * lines < kRsScLines && (q + 4 * i) * lines < lines_left;
-            const int voff = in ? s_lane + 16 * (q + 4 * i) : (1 << 30);
+            const int voff = in ? s_lane + 16 * (q + 4 * i) : kRsPast;
             if constexpr (SLD == 2) {
 #pragma unroll
               for (int d = 0; d < 4; ++d) {
-                const uint32_t lo = __builtin_amdgcn_raw_buffer_load_b16(rs, voff + 4 * d, so + c * 16 * G * SB, 0);
-                const uint32_t hi = __builtin_amdgcn_raw_buffer_load_b16(rs, voff + 4 * d + 2, so + c * 16 * G * SB, 0);
+                const uint32_t lo = __builtin_amdgcn_raw_buffer_load_b16(rs, voff + 4 * d, so + c * tile * G * SB, 0);
+                const uint32_t hi = __builtin_amdgcn_raw_buffer_load_b16(rs, voff + 4 * d + 2, so + c * tile * G * SB, 0);
                 sl.s[c][i][d] = lo | (hi << 16);
               }
             } else if constexpr (SLD == 4) {
 #pragma unroll
               for (int d = 0; d < 4; ++d)
-                sl.s[c][i][d] = __builtin_amdgcn_raw_buffer_load_b32(rs, voff + 4 * d, so + c * 16 * G * SB,
+                sl.s[c][i][d] = __builtin_amdgcn_raw_buffer_load_b32(rs, voff + 4 * d, so + c * tile * G * SB,
                                                                      0);
             } else {
               sl.s[c][i] = __builtin_amdgcn_raw_buffer_load_b128(rs, voff, so + c * 16 * G * SB,
@@ -523,6 +518,19 @@ __device__ __forceinline__ void stream_body(const RsArgs& p) {
         for (int c = 0; c < 2; ++c)
 #pragma unroll
           for (int i = 0; i < F::kScLoads; ++i) sc_lds[wave][c][i * 64 + lane] = sl.s[c][i];
+        if constexpr (PADK) {
+          // scales g0 .. g1 - 1 of the block lie past K: zeroed there (masking
+          // the loaded registers instead cost INT4 5 %)
+          const int g0 = G - ((s * (Ks >> 5) + cl * 8) >> glog);
+          const int g1 = ((min(kRsScLines, nl - cl) * 8 - 1) >> glog) + 1;
+          for (int t = lane; t < (g1 - g0) * 32; t += 64) {
+            const int g = g0 + (t >> 5), c = t & 1, col = (t >> 1) & 15;
+            if constexpr (FMT == kFmtInt4)
+              reinterpret_cast<uint16_t*>(&sc_lds[wave][c][(g >> 3) * 16 + col])[g & 7] = 0;
+            else
+              reinterpret_cast<uint8_t*>(&sc_lds[wave][c][(g >> 4) * 16 + col])[g & 15] = 0;
+          }
+        }
       }
       u32x4 sv[2];     // INT4: the line's 8 bf16 scales
       uint2 sb[2];     // MXFP4: the line's 8 e8m0 bytes
