@@ -284,3 +284,53 @@ def test_stage_entry_keeps_padded_shapes_on_the_stream_kernel():
                           _lib._XK_INT4_TEST_FORCE_STREAM)
     assert _rc("xk_moe_int4_w4a16_gemm", FAKE, 0, 4, 64, FAKE, FAKE, 2, 16, 32, FAKE, 2, None, 0, FAKE, FAKE,
                FAKE, 1 << 10, None, 0, None) == _lib.XK_ERR_INVALID  # internal, not a caller's
+
+
+def _mxfp4_tiles(M, E, hidden, ispp, top_k, f32=False, experts=0):
+    """Which projections (gate/up, down) run on the tile kernel off the stream path."""
+    lib, i64 = _lib.load(), ctypes.c_int64
+    gate_up, down = lib["_ZN2xk18mxfp4_tile_gate_upEllllb"], lib["_ZN2xk15mxfp4_tile_downEllll"]
+    gate_up.restype = down.restype = ctypes.c_bool
+    local = -(-M * top_k * E // experts) if experts else M * top_k
+    sizes = [i64(x) for x in (local, E, hidden, ispp)]
+    return gate_up(*sizes, ctypes.c_bool(f32)), down(*sizes)
+
+
+@pytest.mark.parametrize("M,E,hidden,ispp,k,f32,experts,want", [
+    # the tile kernel took up to twice the passes' time at these (measured)
+    (1, 256, 4096, 512, 6, True, 0, (False, False)),
+    (16, 64, 2048, 1408, 8, True, 0, (False, False)),
+    (60, 32, 2880, 2880, 4, True, 0, (False, False)),
+    (120, 32, 2848, 2912, 4, False, 0, (False, False)),
+    (16, 1024, 2048, 512, 8, False, 0, (False, False)),
+    (107, 32, 4096, 512, 6, False, 256, (False, False)),
+    (512, 32, 4096, 512, 6, False, 256, (False, False)),
+    # and less from here on
+    (128, 256, 4096, 512, 6, True, 0, (True, False)),
+    (400, 64, 2048, 1408, 8, True, 0, (True, True)),
+    (400, 32, 2848, 2912, 4, False, 0, (True, True)),
+    (2048, 32, 4096, 512, 6, False, 256, (True, False)),
+    (4096, 256, 4096, 512, 6, False, 0, (True, True)),
+    (64, 128, 7168, 2048, 8, True, 0, (True, True)),
+])
+def test_mxfp4_kernel_of_each_projection(M, E, hidden, ispp, k, f32, experts, want):
+    assert _mxfp4_tiles(M, E, hidden, ispp, k, f32, experts) == want
+
+
+def test_mxfp4_workspace_serves_smaller_batches():
+    """The bytes never fall with the batch, also across the limits of the stream
+    path, and the halves of a batch past the tile kernel's 2^31 bytes fit what
+    the whole batch asks for."""
+    q = lambda *a: _lib.query("xk_moe_mxfp4_workspace_bytes", *a)
+    for k, E, hidden, ispp in ((6, 256, 4096, 512), (8, 64, 2048, 1408), (4, 32, 2880, 2880), (1, 4, 96, 64),
+                               (8, 600, 256, 128)):
+        sizes = [q(M, k, E, hidden, ispp) for M in range(1, 1500)]
+        assert sizes == sorted(sizes)
+        M = -(-2**31 // (2 * max(hidden, k * ispp)))  # the first batch past the limit
+        for whole in (M, M + 1, 3 * M + 1):
+            part = whole
+            while part * 2 * max(hidden, k * ispp) >= 2**31:
+                part = (part + 1) // 2
+            last = whole % part or part
+            assert q(part, k, E, hidden, ispp) <= q(whole, k, E, hidden, ispp)
+            assert q(last, k, E, hidden, ispp) <= q(whole, k, E, hidden, ispp)

@@ -61,6 +61,11 @@ int topk_softmax_max_experts();
 int launch_topk_softmax(const void* logits, int dtype, int64_t M, int64_t E, int64_t k,
                         int renorm, float* w, int32_t* ids, hipStream_t stream);
 int mxfp4_block_size();
+int launch_mxfp4_stage(int stage, const void* A, int a_dtype, const uint8_t* w,
+                       const uint8_t* ws, const uint16_t* bias, int64_t E, int64_t K,
+                       int64_t wrows, int64_t ncols, const int32_t* sorted_ids,
+                       const int32_t* offsets, int64_t numel, int64_t top_k, float limit,
+                       uint16_t* act, uint16_t* rows, hipStream_t stream);
 int launch_activations_to_bf16(const float* a, int64_t n, uint16_t* out, hipStream_t stream);
 bool small_int4_ok(int a_dtype, int64_t M, int64_t top_k, int64_t E, int64_t N, int64_t K, int group_size,
                    const void* A, const void* packed, const void* scale);
@@ -437,16 +442,18 @@ int xk_moe_topk_softmax(const void* gating_output, int32_t dtype, int64_t M, int
 namespace {
 
 // The MXFP4 pipeline: both projections through the stream kernel (bf16
-// activations, few routed rows per expert, sizes multiples of 64), else
-// through the tile kernel.
+// activations, few routed rows per expert, sizes multiples of 64), else each
+// through 32-row passes or the tile kernel (mxfp4_tile_gate_up, _down).
 // Workspace after the align scratch: act [numel, ispp] bf16, then the stream
 // path's down planes [S1, numel, hidden] fp32 and gate/up planes [S0, numel,
-// 2 ispp] fp32, or the tile path's down rows [numel, hidden] bf16, its bf16
-// activations [M, hidden] (fp32 calls) and its two tile queues.
-// Routed rows per expert (on average) from which the tile kernel runs: E = 256,
-// hidden 4096, ispp 512, top_k 6, stream vs tile 288 vs 322 us at 14 rows, 400
-// vs 343 at 23; E = 64, hidden 2048, ispp 1408, top_k 8: 123 vs 173 at 19 rows,
-// 226 vs 193 at 50.
+// 2 ispp] fp32, or the other kernels' down rows [numel, hidden] bf16, the bf16
+// activations [M, hidden] (fp32 calls) and the two tile queues.
+// Routed rows per expert (on average) up to which the stream kernel runs.
+// One line for shapes that cross at different places, the stream kernel against
+// the others: E = 256, hidden 4096, ispp 512, top_k 6: 353 vs 304 us at 20 rows;
+// E = 32, hidden = ispp = 2880, top_k 4: 183 vs 175 at 20, 213 vs 233 at 28, 283
+// vs 247 at 40; E = 64, hidden 2048, ispp 1408, top_k 8 crosses last: 124 vs 137
+// at 20, 134 vs 165 at 24, 161 vs 165 at 32, 198 vs 184 at 40.
 constexpr int64_t kMxStreamRowsPerExpert = 20;
 
 // Whether a batch's activations fit one tile launch (2^31-byte buffers).
@@ -459,10 +466,10 @@ struct Mxfp4Plan {
   int s0, s1;
   int64_t act, down, gu, abf, queue, total;
   Mxfp4Plan(int64_t M, int64_t top_k, int64_t E, int64_t hidden, int64_t ispp, int a_dtype,
-            bool tile_only = false) {
+            bool no_stream = false) {
     const int64_t numel = M * top_k;
     AlignScratch al(numel, int(E), mxfp4_block_size());
-    stream = !tile_only && a_dtype == XK_DT_BF16 && numel > 0 && numel < kMxStreamRowsPerExpert * E &&
+    stream = !no_stream && a_dtype == XK_DT_BF16 && numel > 0 && numel < kMxStreamRowsPerExpert * E &&
              mxfp4_rs_ok(M, hidden, 2 * ispp, E, numel) &&
              mxfp4_rs_ok(numel, ispp, hidden, E, numel);
     s0 = stream ? mxfp4_rs_slices(hidden, 2 * ispp, numel, E) : 0;
@@ -475,6 +482,45 @@ struct Mxfp4Plan {
     total = stream ? gu + round_up(s0 * numel * 2 * ispp * 4) : queue + round_up(2 * tile_queue_bytes());
   }
 };
+
+// Slots expected on the E local experts: under an expert map their share of the
+// global ones, so that a rank of an expert-parallel group picks the kernels the
+// dense call picks for the same rows per expert.
+int64_t mxfp4_local_slots(int64_t numel, int64_t E, const void* expert_map, int64_t num_global) {
+  return expert_map != nullptr && num_global > E ? cdiv(numel * E, num_global) : numel;
+}
+
+// The kernel of each projection off the stream path: 128-row tiles (true) or
+// 32-row passes (mxfp4_stream_gemm). A pass costs each workgroup its weights
+// once per 32 rows; a tile costs a fixed start and end (a ticket, the first
+// chunk's loads, the stores) and needs many tiles on the 512 places, which rows,
+// experts, columns and the length of the contraction K all bring. Measured per
+// call, the tile's time less the passes':
+//   gate/up, bf16: E = 32, hidden 2848, ispp 2912: +35 us at 15 rows per expert,
+//     +9 at 25, -28 at 32; 32 of 256 experts, hidden 4096, ispp 512: +22 at 12,
+//     -1 at 24, -18 at 32; E = 1024, hidden 2048, ispp 512: +9 at 256 slots, -23
+//     at 512, -49 at 1,024; E = 600, hidden 7168, ispp 2048: -84 at 64 slots.
+//   gate/up, fp32 (the passes read twice the bytes): E = 64, hidden 2048, ispp
+//     1408: +6 at 2 rows per expert, -14 at 16; E = 32, hidden = ispp = 2880: +5
+//     at 2, +17 at 8, -1 at 15; E = 64, hidden 4096, ispp 2048: +2 at 16 slots,
+//     -27 at 32.
+//   down: E = 256, hidden 4096, ispp 512: +27 at 3 rows, +15 at 24, -9 at 32, -37
+//     at 48; 32 of 256 experts +28 at 48, +11 at 96; E = 64, hidden 2048, ispp
+//     1408: +15 at 30, -6 at 50; E = 32, hidden = ispp = 2880: +29 at 15, +1 at
+//     25, -38 at 50; E = 128, hidden 7168, ispp 2048: -35 at 1 row.
+}  // namespace
+namespace xk {
+bool mxfp4_tile_gate_up(int64_t local, int64_t E, int64_t hidden, int64_t ispp, bool f32) {
+  return local >= (f32 ? 14 : 28) * E ||
+         std::min(local, E) * cdiv(ispp, 128) * hidden * hidden >= (int64_t(1) << 33);
+}
+bool mxfp4_tile_down(int64_t local, int64_t E, int64_t hidden, int64_t ispp) {
+  const int64_t col_tiles = cdiv(hidden, 256);
+  return (local >= 28 * E && local * col_tiles * ispp >= 28000000) ||
+         std::min(local, E) * col_tiles * ispp * ispp >= (int64_t(1) << 32);
+}
+}  // namespace xk
+namespace {
 
 // Tokens of the largest part of a batch that one tile launch takes.
 int64_t mxfp4_tile_tokens(int64_t M, int64_t top_k, int64_t hidden, int64_t ispp) {
@@ -583,18 +629,25 @@ int xk_moe_mxfp4(const void* A, int32_t a_dtype, int64_t M, int64_t hidden, cons
                                int(E), expert_map, num_global_experts, out, a_dtype, plan.s1, stream,
                                b2, 1);
   }
+  const int64_t local = mxfp4_local_slots(numel, E, expert_map, num_global_experts);
+  const bool tile_gu = mxfp4_tile_gate_up(local, E, hidden, ispp, a_dtype == XK_DT_FP32);
+  const bool tile_down = mxfp4_tile_down(local, E, hidden, ispp);
+  uint16_t* rows = at<uint16_t>(workspace, plan.down);
   const uint16_t* a16 = static_cast<const uint16_t*>(A);
-  if (a_dtype == XK_DT_FP32) {
+  if (tile_gu && a_dtype == XK_DT_FP32) {
     uint16_t* abf = at<uint16_t>(workspace, plan.abf);
     if ((rc = launch_activations_to_bf16(static_cast<const float*>(A), M * hidden, abf, stream))) return rc;
     a16 = abf;
   }
-  uint16_t* rows = at<uint16_t>(workspace, plan.down);
-  rc = launch_mxfp4_tile(0, a16, M, hidden, w13, w13_scale, b13, E, 2 * ispp, sorted, offsets, numel, top_k,
-                         swiglu_limit, act, queue, stream);
+  rc = !tile_gu ? launch_mxfp4_stage(0, A, a_dtype, w13, w13_scale, b13, E, hidden, 2 * ispp, ispp, sorted, offsets,
+                                     numel, top_k, swiglu_limit, act, nullptr, stream)
+                : launch_mxfp4_tile(0, a16, M, hidden, w13, w13_scale, b13, E, 2 * ispp, sorted, offsets, numel,
+                                    top_k, swiglu_limit, act, queue, stream);
   if (rc) return rc;
-  rc = launch_mxfp4_tile(1, act, numel, ispp, w2, w2_scale, b2, E, hidden, sorted, offsets, numel, 1, 0.f, rows,
-                         queue + nq, stream);
+  rc = !tile_down ? launch_mxfp4_stage(1, act, XK_DT_BF16, w2, w2_scale, b2, E, ispp, hidden, hidden, sorted, offsets,
+                                       numel, 1, 0.f, nullptr, rows, stream)
+                  : launch_mxfp4_tile(1, act, numel, ispp, w2, w2_scale, b2, E, hidden, sorted, offsets, numel, 1,
+                                      0.f, rows, queue + nq, stream);
   if (rc) return rc;
   return launch_topk_combine_bf16(rows, M, top_k, hidden, topk_w, mul_routed_weight, topk_ids, int(E), expert_map,
                                   num_global_experts, out, a_dtype, stream);
