@@ -67,8 +67,8 @@ int launch_mxfp4_stage(int stage, const void* A, int a_dtype, const uint8_t* w,
                        const int32_t* offsets, int64_t numel, int64_t top_k, float limit,
                        uint16_t* act, uint16_t* rows, hipStream_t stream);
 int launch_activations_to_bf16(const float* a, int64_t n, uint16_t* out, hipStream_t stream);
-bool small_int4_ok(int a_dtype, int64_t M, int64_t top_k, int64_t E, int64_t N, int64_t K, int group_size,
-                   const void* A, const void* packed, const void* scale);
+bool small_int4_ok(int a_dtype, int64_t M, int64_t top_k, int64_t local_slots, int64_t E, int64_t N, int64_t K,
+                   int group_size, const void* A, const void* packed, const void* scale);
 int launch_small_int4(const uint16_t* A, int64_t M, int64_t K, const int32_t* packed, const uint16_t* scale,
                       int64_t E, int64_t N, const int32_t* topk_ids, const float* weights, int64_t top_k,
                       const int32_t* emap, int num_global, uint16_t* out, hipStream_t stream);
@@ -120,6 +120,13 @@ struct AlignScratch {
     total = o;
   }
 };
+
+// Slots expected on the E local experts: under an expert map their share of the
+// global ones, so that a rank of an expert-parallel group picks the kernels the
+// dense call picks for the same rows per expert.
+int64_t local_slots(int64_t numel, int64_t E, const void* expert_map, int64_t num_global) {
+  return expert_map != nullptr && num_global > E ? cdiv(numel * E, num_global) : numel;
+}
 
 template <typename T> T* at(void* base, int64_t off) {
   return reinterpret_cast<T*>(static_cast<char*>(base) + off);
@@ -312,7 +319,8 @@ int xk_moe_int4_w4a16(const void* A, int32_t a_dtype, int64_t M, int64_t K,
   if (workspace == nullptr || workspace_bytes < need)
     return set_error(XK_ERR_WORKSPACE, "int4: workspace %lld B < %lld B",
                      (long long)workspace_bytes, (long long)need);
-  if (flags == 0 && small_int4_ok(a_dtype, M, top_k, E, N, K, group_size, A, packed, scale))
+  if (flags == 0 && small_int4_ok(a_dtype, M, top_k, local_slots(M * top_k, E, expert_map, num_global_experts), E,
+                                  N, K, group_size, A, packed, scale))
     return launch_small_int4(static_cast<const uint16_t*>(A), M, K, packed, scale, E, N, topk_ids,
                              mul_routed_weight ? topk_w : nullptr, top_k, expert_map, num_global_experts,
                              static_cast<uint16_t*>(out), stream);
@@ -483,13 +491,6 @@ struct Mxfp4Plan {
   }
 };
 
-// Slots expected on the E local experts: under an expert map their share of the
-// global ones, so that a rank of an expert-parallel group picks the kernels the
-// dense call picks for the same rows per expert.
-int64_t mxfp4_local_slots(int64_t numel, int64_t E, const void* expert_map, int64_t num_global) {
-  return expert_map != nullptr && num_global > E ? cdiv(numel * E, num_global) : numel;
-}
-
 // The kernel of each projection off the stream path: 128-row tiles (true) or
 // 32-row passes (mxfp4_stream_gemm). A pass costs each workgroup its weights
 // once per 32 rows; a tile costs a fixed start and end (a ticket, the first
@@ -629,7 +630,7 @@ int xk_moe_mxfp4(const void* A, int32_t a_dtype, int64_t M, int64_t hidden, cons
                                int(E), expert_map, num_global_experts, out, a_dtype, plan.s1, stream,
                                b2, 1);
   }
-  const int64_t local = mxfp4_local_slots(numel, E, expert_map, num_global_experts);
+  const int64_t local = local_slots(numel, E, expert_map, num_global_experts);
   const bool tile_gu = mxfp4_tile_gate_up(local, E, hidden, ispp, a_dtype == XK_DT_FP32);
   const bool tile_down = mxfp4_tile_down(local, E, hidden, ispp);
   uint16_t* rows = at<uint16_t>(workspace, plan.down);

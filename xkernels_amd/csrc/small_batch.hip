@@ -18,7 +18,7 @@
 //   * its waves split (expert, 512-k unit) pairs evenly, each with the next
 //     unit's 16-byte loads in flight while one is contracted.
 // Per call, stream path -> here: INT4 at N = 4096, K = 7168, 1 / 2 / 4 / 8 tokens
-// 46 -> 31, 67 -> 57, 93 -> 86, 124 -> 123 us; N = 7168, K = 2048, 1 / 4 / 8
+// 46 -> 31, 67 -> 57, 93 -> 86, 124 -> 123 us (fewer columns: small_int4_faster); N = 7168, K = 2048, 1 / 4 / 8
 // tokens 25.5 -> 19, 51 -> 48, 67 -> 68 us; MXFP4, 1 / 4 / 8 tokens 28.8 -> 19.1,
 // 39 -> 28, 53.5 -> 53 us. From 8 tokens on the experts' weights hide the
 // latencies either way.
@@ -370,12 +370,27 @@ bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0;
 
 }  // namespace
 
+// A workgroup of small_int4 walks the weights of 16 columns for every expert of
+// the batch, so its time grows with experts x K, and only many columns (N / 16
+// workgroups) make the calls that the stream kernel, which splits experts x
+// columns over all CUs, does not do sooner. With U = experts x K / 8192 (512-k
+// units per wave of 16) the call takes about 2 + 3 U us against 18 + U N / 1250.
+// E = 64, top_k 8, stream vs here: K = 7168, N = 1024: 1 token 27 vs 25 us, 3
+// tokens 33 vs 55, 6 tokens 44 vs 97; N = 64: 1 token 24 vs 24, 6 tokens 25 vs 92;
+// K = 2048, N = 512: 1 token 19 vs 13, 6 tokens 20 vs 34; N = 4096: K = 7168, E =
+// 48, 6 tokens 109 vs 104, K = 10240 161 vs 167.
+bool small_int4_faster(int64_t slots, int64_t E, int64_t N, int64_t K) {
+  const int64_t experts_k = std::min(slots, E) * K;
+  return experts_k * (3750 - N) < 220000000 && experts_k <= 45 * 8192;
+}
+
 // Batches the one-launch INT4 kernel takes: bf16 activations, groups of 32, at
 // most 6 tokens and 64 slots, K a multiple of 512, N of 16, 16-byte aligned
-// pointers, the tokens' activations in the LDS.
-bool small_int4_ok(int a_dtype, int64_t M, int64_t top_k, int64_t E, int64_t N, int64_t K, int group_size,
-                   const void* A, const void* packed, const void* scale) {
-  return a_dtype == XK_DT_BF16 && group_size == 32 && M >= 1 && M <= kMaxTokens && M * top_k <= kSlots &&
+// pointers, the tokens' activations in the LDS. `local_slots`: the slots
+// expected on the E local experts (all of them without an expert map).
+bool small_int4_ok(int a_dtype, int64_t M, int64_t top_k, int64_t local_slots, int64_t E, int64_t N, int64_t K,
+                   int group_size, const void* A, const void* packed, const void* scale) {
+  return small_int4_faster(local_slots, E, N, K) && a_dtype == XK_DT_BF16 && group_size == 32 && M >= 1 && M <= kMaxTokens && M * top_k <= kSlots &&
          K % kUnitK == 0 && N % 16 == 0 && N / 16 < (1 << 30) && K < (1 << 24) && E <= 65535 &&
          row_lds(M, K) <= kSmallLds && aligned16(A) && aligned16(packed) && aligned16(scale);
 }
