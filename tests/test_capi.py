@@ -339,14 +339,13 @@ def test_mxfp4_workspace_serves_smaller_batches():
 @pytest.mark.parametrize("M,E,N,K,k,experts,want", [
     (1, 64, 64, 7168, 8, 0, True), (1, 48, 4096, 7168, 8, 0, True), (6, 48, 4096, 7168, 8, 0, True),
     (6, 48, 7168, 2048, 8, 0, True), (6, 48, 7168, 2048, 8, 384, True), (1, 64, 512, 2048, 8, 0, True),
-    (6, 8, 1024, 2048, 2, 0, True),
+    (6, 8, 1024, 2048, 2, 0, True), (6, 4, 256, 7168, 4, 0, True),
     # few columns and many experts: the stream kernel takes a quarter to half the time
     (6, 64, 16, 7168, 8, 0, False), (3, 64, 256, 7168, 8, 0, False), (6, 64, 1024, 7168, 8, 0, False),
-    (6, 64, 512, 2048, 8, 0, False), (2, 64, 256, 14336, 8, 0, False), (6, 64, 4096, 10240, 8, 0, False),
+    (6, 64, 512, 2048, 8, 0, False), (3, 64, 512, 2048, 8, 0, False), (6, 16, 2048, 4096, 4, 0, False), (2, 64, 256, 14336, 8, 0, False), (6, 64, 4096, 10240, 8, 0, False),
 ])
 def test_int4_one_launch_kernel_choice(M, E, N, K, k, experts, want):
     lib, i64, ptr = _lib.load(), ctypes.c_int64, ctypes.c_void_p(256)
     ok = lib["_ZN2xk13small_int4_okEilllllliPKvS1_S1_"]
     ok.restype = ctypes.c_bool
-    local = -(-M * k * E // experts) if experts else M * k
-    assert ok(_lib.XK_DT_BF16, *(i64(x) for x in (M, k, local, E, N, K)), 32, ptr, ptr, ptr) == want
+    assert ok(_lib.XK_DT_BF16, *(i64(x) for x in (M, k, E, experts or E, N, K)), 32, ptr, ptr, ptr) == want

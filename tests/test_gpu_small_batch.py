@@ -2,7 +2,8 @@
 one to six tokens, up to 64 routed slots, duplicated experts within a token,
 dropped slots under an expert map, no routed slot at all, unweighted sums, more
 column blocks than compute units, one 512-k unit and many, and the first sizes
-past their limits (7 tokens, 65 slots), against the oracle."""
+past their limits (7 tokens, 65 slots, more experts than the INT4 kernel takes at
+few columns), against the oracle."""
 from __future__ import annotations
 
 import pytest
@@ -15,7 +16,8 @@ from xkernels_amd import (Backend, fused_moe_int4_w4a16, fused_moe_mxfp4, make_m
 
 pytestmark = pytest.mark.gpu
 
-CASES = [(1, 8, 1), (1, 8, 8), (2, 4, 4), (3, 48, 8), (6, 16, 8), (6, 3, 10), (1, 64, 64), (7, 8, 8), (5, 16, 13)]
+CASES = [(1, 8, 1), (1, 8, 8), (2, 4, 4), (3, 48, 8), (6, 16, 8), (6, 3, 10), (1, 64, 64), (7, 8, 8), (5, 16, 13),
+         (1, 3, 64), (2, 12, 32)]
 
 
 def _route(M, E, k, seed):

@@ -67,7 +67,7 @@ int launch_mxfp4_stage(int stage, const void* A, int a_dtype, const uint8_t* w,
                        const int32_t* offsets, int64_t numel, int64_t top_k, float limit,
                        uint16_t* act, uint16_t* rows, hipStream_t stream);
 int launch_activations_to_bf16(const float* a, int64_t n, uint16_t* out, hipStream_t stream);
-bool small_int4_ok(int a_dtype, int64_t M, int64_t top_k, int64_t local_slots, int64_t E, int64_t N, int64_t K,
+bool small_int4_ok(int a_dtype, int64_t M, int64_t top_k, int64_t E, int64_t routed, int64_t N, int64_t K,
                    int group_size, const void* A, const void* packed, const void* scale);
 int launch_small_int4(const uint16_t* A, int64_t M, int64_t K, const int32_t* packed, const uint16_t* scale,
                       int64_t E, int64_t N, const int32_t* topk_ids, const float* weights, int64_t top_k,
@@ -319,8 +319,9 @@ int xk_moe_int4_w4a16(const void* A, int32_t a_dtype, int64_t M, int64_t K,
   if (workspace == nullptr || workspace_bytes < need)
     return set_error(XK_ERR_WORKSPACE, "int4: workspace %lld B < %lld B",
                      (long long)workspace_bytes, (long long)need);
-  if (flags == 0 && small_int4_ok(a_dtype, M, top_k, local_slots(M * top_k, E, expert_map, num_global_experts), E,
-                                  N, K, group_size, A, packed, scale))
+  if (flags == 0 && small_int4_ok(a_dtype, M, top_k, E,
+                                  expert_map != nullptr && num_global_experts > E ? num_global_experts : E, N, K,
+                                  group_size, A, packed, scale))
     return launch_small_int4(static_cast<const uint16_t*>(A), M, K, packed, scale, E, N, topk_ids,
                              mul_routed_weight ? topk_w : nullptr, top_k, expert_map, num_global_experts,
                              static_cast<uint16_t*>(out), stream);

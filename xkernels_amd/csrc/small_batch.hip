@@ -23,6 +23,7 @@
 // 39 -> 28, 53.5 -> 53 us. From 8 tokens on the experts' weights hide the
 // latencies either way.
 #include <algorithm>
+#include <cmath>
 
 #include "int4_common.h"
 
@@ -370,29 +371,33 @@ bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0;
 
 }  // namespace
 
-// A workgroup of small_int4 walks the weights of 16 columns for every expert of
-// the batch, so its time grows with experts x K, and only many columns (N / 16
-// workgroups) make the calls that the stream kernel, which splits experts x
-// columns over all CUs, does not do sooner. With U = experts x K / 8192 (512-k
-// units per wave of 16) the call takes about 2 + 3 U us against 18 + U N / 1250.
-// E = 64, top_k 8, stream vs here: K = 7168, N = 1024: 1 token 27 vs 25 us, 3
-// tokens 33 vs 55, 6 tokens 44 vs 97; N = 64: 1 token 24 vs 24, 6 tokens 25 vs 92;
-// K = 2048, N = 512: 1 token 19 vs 13, 6 tokens 20 vs 34; N = 4096: K = 7168, E =
-// 48, 6 tokens 109 vs 104, K = 10240 161 vs 167.
-bool small_int4_faster(int64_t slots, int64_t E, int64_t N, int64_t K) {
-  const int64_t experts_k = std::min(slots, E) * K;
-  return experts_k * (3750 - N) < 220000000 && experts_k <= 45 * 8192;
+// A workgroup of small_int4 walks the weights of 16 columns for every expert X of
+// the batch, about 2 + X (K + 1000) / 3000 us whatever N is; the stream kernel
+// splits experts x columns over all CUs, about 14 + K / 1300 + X N K / 10^7 us. So
+// it runs for few experts, or for so many columns that the weights take longer
+// than their latencies (up to a size where the stream kernel reads them a little
+// better). E = 64, top_k 8, stream vs here: K = 7168, N = 1024: 1 token 27 vs 25
+// us, 3 tokens 33 vs 55, 6 tokens 44 vs 97; N = 64: 1 token 24 vs 24, 6 tokens 25
+// vs 92; K = 2048, N = 512: 1 token 19 vs 13, 3 tokens 19 vs 23, 6 tokens 20 vs
+// 34; N = 4096: E = 48, K = 7168, 6 tokens 107 vs 101, K = 10240 161 vs 167.
+bool small_int4_faster(int64_t M, int64_t top_k, int64_t E, int64_t routed, int64_t N, int64_t K) {
+  // local experts that `M` tokens' slots are expected to reach
+  const double miss = 1.0 - double(std::min(top_k, routed)) / double(routed);
+  const double experts = double(E) * (1.0 - std::pow(miss, double(M)));
+  return experts * double(K + 1000) <= 38000.0 + 3.85 * double(K) ||
+         (N * K >= 3296 * (K + 1000) && experts * double(K) <= 300000.0);
 }
 
 // Batches the one-launch INT4 kernel takes: bf16 activations, groups of 32, at
 // most 6 tokens and 64 slots, K a multiple of 512, N of 16, 16-byte aligned
-// pointers, the tokens' activations in the LDS. `local_slots`: the slots
-// expected on the E local experts (all of them without an expert map).
-bool small_int4_ok(int a_dtype, int64_t M, int64_t top_k, int64_t local_slots, int64_t E, int64_t N, int64_t K,
+// pointers, the tokens' activations in the LDS. `routed`: the experts that the
+// ids range over (under an expert map more than the E local ones).
+bool small_int4_ok(int a_dtype, int64_t M, int64_t top_k, int64_t E, int64_t routed, int64_t N, int64_t K,
                    int group_size, const void* A, const void* packed, const void* scale) {
-  return small_int4_faster(local_slots, E, N, K) && a_dtype == XK_DT_BF16 && group_size == 32 && M >= 1 && M <= kMaxTokens && M * top_k <= kSlots &&
+  return a_dtype == XK_DT_BF16 && group_size == 32 && M >= 1 && M <= kMaxTokens && M * top_k <= kSlots &&
          K % kUnitK == 0 && N % 16 == 0 && N / 16 < (1 << 30) && K < (1 << 24) && E <= 65535 &&
-         row_lds(M, K) <= kSmallLds && aligned16(A) && aligned16(packed) && aligned16(scale);
+         row_lds(M, K) <= kSmallLds && aligned16(A) && aligned16(packed) && aligned16(scale) &&
+         small_int4_faster(M, top_k, E, routed, N, K);
 }
 
 int launch_small_int4(const uint16_t* A, int64_t M, int64_t K, const int32_t* packed, const uint16_t* scale,
