@@ -349,3 +349,17 @@ def test_int4_one_launch_kernel_choice(M, E, N, K, k, experts, want):
     ok = lib["_ZN2xk13small_int4_okEilllllliPKvS1_S1_"]
     ok.restype = ctypes.c_bool
     assert ok(_lib.XK_DT_BF16, *(i64(x) for x in (M, k, E, experts or E, N, K)), 32, ptr, ptr, ptr) == want
+
+
+@pytest.mark.parametrize("M,E,hidden,ispp,k,want", [
+    (1, 256, 4096, 512, 6, True), (6, 256, 4096, 512, 6, True), (3, 64, 4096, 1024, 8, True),
+    (5, 256, 7168, 512, 8, True), (2, 64, 7168, 2048, 8, True),
+    # rows that leave a CU one workgroup: the stream kernel is faster
+    (6, 256, 7168, 512, 8, False), (4, 64, 4096, 1024, 8, False), (4, 32, 2048, 2048, 4, False),
+    (7, 256, 4096, 512, 6, False), (1, 256, 4096, 544, 6, False), (5, 64, 512, 512, 13, False),
+])
+def test_mxfp4_small_kernels_choice(M, E, hidden, ispp, k, want):
+    lib, i64, ptr = _lib.load(), ctypes.c_int64, ctypes.c_void_p(256)
+    ok = lib["_ZN2xk14small_mxfp4_okEilllllPKvS1_S1_S1_S1_"]
+    ok.restype = ctypes.c_bool
+    assert ok(_lib.XK_DT_BF16, *(i64(x) for x in (M, k, E, hidden, ispp)), ptr, ptr, ptr, ptr, ptr) == want

@@ -417,12 +417,19 @@ int launch_small_int4(const uint16_t* A, int64_t M, int64_t K, const int32_t* pa
   return XK_OK;
 }
 
-// MXFP4: the same, for hidden and ispp multiples of 512.
+// MXFP4: the same, for hidden and ispp multiples of 512, with rows in the LDS that
+// leave room for two workgroups a CU; the down projection loads a row per slot in
+// every workgroup, which costs it more from 3 tokens on. Stream vs here: E = 256, hidden 7168, ispp
+// 512, top_k 8, 5 tokens (70 KiB) 64 vs 62 us, 6 tokens (84 KiB) 73 vs 95; E = 64,
+// hidden 4096, ispp 1024, top_k 8, 3 tokens (down 48 KiB) 43 vs 42, 4 tokens (64.5
+// KiB) 50 vs 53, 6 tokens (97 KiB) 62 vs 73; hidden 7168, ispp 2048, 2 tokens
+// (64.3 KiB) 84 vs 79.
+constexpr int64_t kSmallGateUpLds = 72 * 1024, kSmallDownLds = 64 * 1024;
 bool small_mxfp4_ok(int a_dtype, int64_t M, int64_t top_k, int64_t E, int64_t hidden, int64_t ispp, const void* A,
                     const void* w13, const void* w13_scale, const void* w2, const void* w2_scale) {
   return a_dtype == XK_DT_BF16 && M >= 1 && M <= kMaxTokens && M * top_k <= kSlots && hidden % kUnitK == 0 &&
          ispp % kUnitK == 0 && hidden < (1 << 24) && ispp < (1 << 24) && E <= 1024 &&
-         row_lds(M, hidden) <= kSmallLds && row_lds(M * top_k, ispp) <= kSmallLds && aligned16(A) &&
+         row_lds(M, hidden) <= kSmallGateUpLds && row_lds(M * top_k, ispp) <= (M <= 2 ? kSmallGateUpLds : kSmallDownLds) && aligned16(A) &&
          aligned16(w13) && aligned16(w13_scale) && aligned16(w2) && aligned16(w2_scale);
 }
 
