@@ -149,3 +149,17 @@ def test_16_lane_rows_edges(M, E, k, dt, dev):
     for rows in (g[:M], g[1:]):  # the second starts at another alignment for odd E
         _check(rows, k, True)
         _check(rows, k, False)
+
+
+def test_more_rows_than_16_lane_rows_take(dev):
+    """2^28 rows: 16 lanes for each would pass the 2^32 threads a launch takes."""
+    from xkernels_amd import topk_softmax
+
+    M = (1 << 28) + 3
+    g = torch.zeros(M, 2, dtype=torch.bfloat16, device=dev)
+    g[1::2, 1] = 1.0
+    w, ids = topk_softmax(g, 1, renormalize=False, backend=Backend.HIP)
+    assert int(ids.sum(dtype=torch.int64)) == M // 2 and bool((ids[1::2] == 1).all())
+    want = torch.tensor([0.5, 0.7310585786300049], device=dev)  # softmax of (0, 0) and (0, 1)
+    for i in (0, 1):
+        assert float((w[i::2] - want[i]).abs().max()) < 1e-6

@@ -331,7 +331,9 @@ hipError_t launch_rows16(const void* logits, int64_t M, int E, int k, int renorm
 template <typename T>
 hipError_t launch_typed(const void* logits, int64_t M, int E, int k, int renorm, float* w,
                         int32_t* ids, hipStream_t stream) {
-  if (k <= 16 && E <= 512 && M < (int64_t(1) << 32)) {
+  // a launch takes fewer than 2^32 threads (16 a row here; the kernels below
+  // loop over the rows)
+  if (k <= 16 && E <= 512 && cdiv(M, kTsThreads / 16) * kTsThreads < (int64_t(1) << 32)) {
     if (E <= 128) return launch_rows16<T, 1>(logits, M, E, k, renorm, w, ids, stream);
     if (E <= 256) return launch_rows16<T, 2>(logits, M, E, k, renorm, w, ids, stream);
     return launch_rows16<T, 4>(logits, M, E, k, renorm, w, ids, stream);
