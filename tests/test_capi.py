@@ -277,7 +277,7 @@ def test_stage_entry_keeps_padded_shapes_on_the_stream_kernel():
     the tile kernel, the stage entry the stream kernel, whose plane count it
     answers and whose calls may come without align outputs."""
     q = lambda name, *a: _lib.query(name, *a)
-    for N, K in ((2880, 2880), (4096, 7200), (48, 2048)):
+    for N, K in ((2880, 2880), (4096, 7200), (3088, 2048)):
         assert q("xk_moe_int4_kernel", 600, 4, 48, N, K, _lib.XK_DT_BF16, 32, 0, 0) == 2
         parts = q("xk_moe_int4_gemm_parts", 600, 4, 48, N, K, _lib.XK_DT_BF16, 32, 0)
         assert parts == q("xk_moe_int4_gemm_parts", 600, 4, 48, N, K, _lib.XK_DT_BF16, 32,
@@ -363,3 +363,28 @@ def test_mxfp4_small_kernels_choice(M, E, hidden, ispp, k, want):
     ok = lib["_ZN2xk14small_mxfp4_okEilllllPKvS1_S1_S1_S1_"]
     ok.restype = ctypes.c_bool
     assert ok(_lib.XK_DT_BF16, *(i64(x) for x in (M, k, E, hidden, ispp)), ptr, ptr, ptr, ptr, ptr) == want
+
+
+@pytest.mark.parametrize("rows,E,N,K,want", [
+    # stream (1) or tile (2) at sizes that are not multiples of 256, rows per expert
+    (33, 48, 2880, 2880, 1), (50, 48, 2880, 2880, 2), (64, 16, 2880, 2880, 1), (100, 16, 2880, 2880, 2),
+    (100, 16, 2880, 1024, 1), (400, 16, 2880, 1024, 2), (42, 8, 2880, 512, 1), (400, 8, 2880, 512, 1),
+    (1600, 8, 2880, 512, 2), (400, 8, 128, 512, 1), (512, 8, 16, 512, 1), (42, 48, 7184, 2048, 2),
+])
+def test_int4_kernel_of_padded_sizes(rows, E, N, K, want):
+    assert _lib.query("xk_moe_int4_kernel", rows * E, 1, E, N, K, _lib.XK_DT_BF16, 32, 0, 0) == want
+    # the same rows on 1 of 8 ranks
+    assert _lib.query("xk_moe_int4_kernel", rows * E, 8, E, N, K, _lib.XK_DT_BF16, 32, 0, 8 * E) == want
+
+
+@pytest.mark.parametrize("rows,E,N,want", [
+    # 256-row (True) or 128-row tiles, rows per expert
+    (18, 48, 4096, False), (100, 48, 4096, False), (133, 48, 4096, True), (256, 48, 4096, False),
+    (683, 48, 4096, True), (25, 48, 7168, False), (180, 48, 7168, True),
+    (18, 16, 2048, True), (100, 16, 2048, True), (400, 16, 2048, True), (18, 64, 512, True), (400, 64, 512, True),
+    (42, 48, 2048, True), (18, 8, 1024, False), (400, 8, 1024, False),
+])
+def test_int4_tile_height(rows, E, N, want):
+    tall = _lib.load()["_ZN2xk15int4_tall_tilesElll"]
+    tall.restype = ctypes.c_bool
+    assert tall(*(ctypes.c_int64(x) for x in (rows * E, E, N))) == want
