@@ -72,6 +72,28 @@ def test_mxfp4_one_token(hidden, ispp, dev):
     assert float((got - want).norm() / want.norm()) < 4e-3
 
 
+@pytest.mark.parametrize("queue_bytes", [32, 256, 1024, 4096])
+@pytest.mark.parametrize("E,N", [(63, 2048), (64, 2048), (64, 2064), (65, 2048), (200, 2048)])
+def test_queue_of_any_spacing_takes_every_tile_once(E, N, queue_bytes, dev):
+    """Tile counts around the 512 places (up to them the tiles are dealt without
+    the queue) and far above, with the XCDs' counters 4 to 128 bytes apart: the
+    rows equal the static deal's bit for bit, from a buffer of NaNs, twice with
+    one queue of old counts."""
+    from tests.test_gpu_int4_prefill import _inputs, _slot_rows
+    K, M = 256, E * 20
+    print(f"tile queue E={E} N={N} bytes={queue_bytes}", flush=True)
+    ids = torch.arange(E, dtype=torch.int32).repeat_interleave(20).reshape(M, 1)
+    A, packed, scale, ids, _ = _inputs(M, E, N, K, ids, seed=E)
+    force = _lib._XK_INT4_TEST_FORCE_TILE
+    static = _slot_rows(A, packed, scale, ids, force)
+    queue = torch.randint(0, 256, (queue_bytes,), dtype=torch.uint8, device=dev)
+    for _ in range(2):
+        queued = _slot_rows(A, packed, scale, ids, force, queue)
+        torch.cuda.synchronize()
+        assert not torch.isnan(queued).any(), "a routed slot row was not written"
+        assert torch.equal(queued, static)
+
+
 @pytest.mark.parametrize("hidden,ispp", [(512, 512), (1024, 160), (96, 512), (32, 32), (2080, 96), (544, 1536)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_mxfp4_tile_edges(hidden, ispp, dtype, dev):

@@ -169,9 +169,9 @@ align_single_wg(const int32_t* __restrict__ ids, int64_t numel, int num_experts,
                 int block_size, const int32_t* __restrict__ emap, int num_global,
                 int64_t max_pad, int64_t max_blocks, int32_t* __restrict__ sorted_ids,
                 int32_t* __restrict__ expert_ids, int32_t* __restrict__ num_post,
-                int32_t* __restrict__ expert_offsets, int* __restrict__ clear, int nclear) {
+                int32_t* __restrict__ expert_offsets, int* __restrict__ clear, int nclear, int clear_stride) {
   extern __shared__ int lds[];
-  if (static_cast<int>(threadIdx.x) < nclear) clear[threadIdx.x] = 0;
+  if (static_cast<int>(threadIdx.x) < nclear) clear[threadIdx.x * clear_stride] = 0;
   const int nw = blockDim.x >> 6;
   int* cnt = lds;                               // [E]   histogram, then cursor
   int* off = cnt + num_experts;                 // [E+1] padded prefix
@@ -196,9 +196,9 @@ align_single_wg(const int32_t* __restrict__ ids, int64_t numel, int num_experts,
 __global__ void __launch_bounds__(256)
 align_count(const int32_t* __restrict__ ids, int64_t numel, int64_t chunk,
             int num_experts, const int32_t* __restrict__ emap, int num_global,
-            int32_t* __restrict__ chunk_cnt, int* __restrict__ clear, int nclear) {
+            int32_t* __restrict__ chunk_cnt, int* __restrict__ clear, int nclear, int clear_stride) {
   extern __shared__ int lds[];
-  if (blockIdx.x == 0 && static_cast<int>(threadIdx.x) < nclear) clear[threadIdx.x] = 0;
+  if (blockIdx.x == 0 && static_cast<int>(threadIdx.x) < nclear) clear[threadIdx.x * clear_stride] = 0;
   for (int i = threadIdx.x; i < num_experts; i += blockDim.x) lds[i] = 0;
   __syncthreads();
   const int64_t begin = blockIdx.x * chunk;
@@ -349,13 +349,13 @@ int64_t align_workspace_bytes(int64_t numel, int num_experts) {
   return nchunks * num_experts * static_cast<int64_t>(sizeof(int32_t));
 }
 
-// `clear`: nclear (at most 64) ints zeroed before the launch's end (a tile
+// `clear`: nclear (at most 64) ints, clear_stride apart, zeroed before the launch's end (a tile
 // kernel's queue: no launch of its own, and no memset in a captured graph).
 int launch_align(const int32_t* ids, int64_t numel, int num_experts, int block_size,
                  const int32_t* emap, int num_global, int32_t* sorted_ids,
                  int32_t* expert_ids, int32_t* num_post, int32_t* expert_offsets,
                  void* workspace, int64_t workspace_bytes, hipStream_t stream, int* clear,
-                 int nclear) {
+                 int nclear, int clear_stride) {
   XK_REQUIRE(num_experts > 0 && num_experts <= kMaxExperts,
              "align: num_experts=%d outside [1, %d]", num_experts, kMaxExperts);
   XK_REQUIRE(block_size > 0 && block_size <= 4096, "align: block_size=%d outside [1, 4096]",
@@ -373,7 +373,7 @@ int launch_align(const int32_t* ids, int64_t numel, int num_experts, int block_s
     const size_t lds = sizeof(int) * (3 * num_experts + 1 + 16 + nw * (num_experts + 1));
     hipLaunchKernelGGL(align_single_wg, dim3(1), dim3(threads), lds, stream, ids, numel,
                        num_experts, block_size, emap, num_global, max_pad, max_blocks,
-                       sorted_ids, expert_ids, num_post, expert_offsets, clear, nclear);
+                       sorted_ids, expert_ids, num_post, expert_offsets, clear, nclear, clear_stride);
     XK_CHECK_LAUNCH("align_single_wg");
     return XK_OK;
   }
@@ -384,7 +384,7 @@ int launch_align(const int32_t* ids, int64_t numel, int num_experts, int block_s
   int32_t* chunk_cnt = static_cast<int32_t*>(workspace);
   hipLaunchKernelGGL(align_count, dim3(nchunks), dim3(256), sizeof(int) * num_experts,
                      stream, ids, numel, kGridChunk, num_experts, emap, num_global,
-                     chunk_cnt, clear, nclear);
+                     chunk_cnt, clear, nclear, clear_stride);
   XK_CHECK_LAUNCH("align_count");
   {
     const int threads = kGridChunk, nw = threads / 64;

@@ -34,7 +34,8 @@ int64_t align_workspace_bytes(int64_t numel, int num_experts);
 int launch_align(const int32_t* ids, int64_t numel, int num_experts, int block_size,
                  const int32_t* emap, int num_global, int32_t* sorted_ids, int32_t* expert_ids,
                  int32_t* num_post, int32_t* expert_offsets, void* workspace,
-                 int64_t workspace_bytes, hipStream_t stream, int* clear = nullptr, int nclear = 0);
+                 int64_t workspace_bytes, hipStream_t stream, int* clear = nullptr, int nclear = 0,
+                 int clear_stride = 1);
 int launch_sum_reduce(const void* y, int y_dtype, int64_t M, int64_t top_k, int64_t H,
                       const void* w, int w_dtype, float scale, void* out, hipStream_t stream);
 int launch_topk_combine(const float* slot_out, int64_t M, int64_t top_k, int64_t N,
@@ -80,10 +81,12 @@ int launch_small_mxfp4(const uint16_t* A, int64_t M, int64_t hidden, const uint8
                        int64_t top_k, const int32_t* emap, int num_global, uint16_t* act, uint16_t* out,
                        hipStream_t stream);
 int64_t tile_queue_bytes();
+int64_t tile_queue_best_bytes();
+int tile_queue_stride(int64_t bytes);
 int launch_mxfp4_tile(int stage, const uint16_t* A, int64_t a_rows, int64_t K, const uint8_t* w,
                       const uint8_t* ws, const uint16_t* bias, int64_t E, int64_t rows,
                       const int32_t* sorted_ids, const int32_t* offsets, int64_t numel,
-                      int64_t a_row_div, float limit, uint16_t* out, int* queue, hipStream_t stream);
+                      int64_t a_row_div, float limit, uint16_t* out, int* queue, int queue_stride, hipStream_t stream);
 int launch_topk_combine_bf16(const uint16_t* rows, int64_t M, int64_t top_k, int64_t N,
                              const float* topk_w, int mul_routed_weight, const int32_t* topk_ids,
                              int num_local, const int32_t* emap, int num_global, void* out,
@@ -382,7 +385,8 @@ int xk_moe_int4_w4a16(const void* A, int32_t a_dtype, int64_t M, int64_t K,
                           at<int32_t>(workspace, al.num_post),
                           at<int32_t>(workspace, al.offsets), at<char>(workspace, al.inner),
                           al.total - al.inner, stream, at<int>(workspace, al.total),
-                          int(tile_queue_bytes() / sizeof(int)));
+                          int(tile_queue_bytes() / sizeof(int)),
+                          tile_queue_stride(round_up(int4_gemm_workspace_bytes(M, K))));
     if (rc) return rc;
     sorted = at<int32_t>(workspace, al.sorted);
     offsets = at<int32_t>(workspace, al.offsets);
@@ -488,7 +492,7 @@ struct Mxfp4Plan {
     gu = down + round_up(stream ? s1 * numel * hidden * 4 : numel * hidden * 2);
     abf = gu;
     queue = abf + round_up(stream || a_dtype == XK_DT_BF16 ? 0 : M * hidden * 2);
-    total = stream ? gu + round_up(s0 * numel * 2 * ispp * 4) : queue + round_up(2 * tile_queue_bytes());
+    total = stream ? gu + round_up(s0 * numel * 2 * ispp * 4) : queue + 2 * tile_queue_best_bytes();
   }
 };
 
@@ -604,13 +608,13 @@ int xk_moe_mxfp4(const void* A, int32_t a_dtype, int64_t M, int64_t hidden, cons
   // the stream kernels route small batches themselves (no align kernel)
   const bool self_route = plan.stream && int4_rs_self_route_ok(numel);
   int* queue = at<int>(workspace, plan.queue);  // the tile path's two
-  const int nq = int(tile_queue_bytes() / sizeof(int));
+  const int nq = int(tile_queue_bytes() / sizeof(int)), queue_stride = tile_queue_stride(tile_queue_best_bytes());
   int rc = XK_OK;
   if (!self_route) {
     rc = launch_align(topk_ids, numel, int(E), mxfp4_block_size(), expert_map, num_global_experts,
                       sorted, at<int32_t>(workspace, al.expert_ids),
                       at<int32_t>(workspace, al.num_post), offsets, at<char>(workspace, al.inner),
-                      al.total - al.inner, stream, plan.stream ? nullptr : queue, plan.stream ? 0 : 2 * nq);
+                      al.total - al.inner, stream, plan.stream ? nullptr : queue, plan.stream ? 0 : 2 * nq, queue_stride);
     if (rc) return rc;
   }
   if (plan.stream) {
@@ -644,12 +648,12 @@ int xk_moe_mxfp4(const void* A, int32_t a_dtype, int64_t M, int64_t hidden, cons
   rc = !tile_gu ? launch_mxfp4_stage(0, A, a_dtype, w13, w13_scale, b13, E, hidden, 2 * ispp, ispp, sorted, offsets,
                                      numel, top_k, swiglu_limit, act, nullptr, stream)
                 : launch_mxfp4_tile(0, a16, M, hidden, w13, w13_scale, b13, E, 2 * ispp, sorted, offsets, numel,
-                                    top_k, swiglu_limit, act, queue, stream);
+                                    top_k, swiglu_limit, act, queue, queue_stride, stream);
   if (rc) return rc;
   rc = !tile_down ? launch_mxfp4_stage(1, act, XK_DT_BF16, w2, w2_scale, b2, E, ispp, hidden, hidden, sorted, offsets,
                                        numel, 1, 0.f, nullptr, rows, stream)
                   : launch_mxfp4_tile(1, act, numel, ispp, w2, w2_scale, b2, E, hidden, sorted, offsets, numel, 1,
-                                      0.f, rows, queue + nq, stream);
+                                      0.f, rows, queue + nq * queue_stride, queue_stride, stream);
   if (rc) return rc;
   return launch_topk_combine_bf16(rows, M, top_k, hidden, topk_w, mul_routed_weight, topk_ids, int(E), expert_map,
                                   num_global_experts, out, a_dtype, stream);

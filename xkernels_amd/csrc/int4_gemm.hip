@@ -100,11 +100,11 @@ bool int4_tile_ok(int a_dtype, int group_size, int64_t M, int64_t K, int64_t N, 
 int launch_int4_tile(const void* A, int64_t K, const int32_t* packed, const uint16_t* scale,
                      int64_t E, int64_t N, int64_t numel, int64_t top_k, int group_size,
                      const int32_t* sorted_ids, const int32_t* offsets, float* slot_out,
-                     int* queue, bool queue_cleared, hipStream_t stream);
+                     int* queue, int queue_stride, bool queue_cleared, hipStream_t stream);
 int launch_int4_prefill(const void* A, int64_t K, const int32_t* packed, const uint16_t* scale,
                         int64_t E, int64_t N, int64_t numel, int64_t top_k, int group_size,
                         const int32_t* sorted_ids, const int32_t* offsets, float* slot_out,
-                        int* queue, bool queue_cleared, hipStream_t stream);
+                        int* queue, int queue_stride, bool queue_cleared, hipStream_t stream);
 
 // Routed rows per expert (on average) from which the tile kernels replace the
 // weight-streaming kernel, which streams every expert's weights once per
@@ -154,6 +154,7 @@ bool int4_tall_tiles(int64_t rows, int64_t E, int64_t N) {
 }
 
 int64_t tile_queue_bytes();
+int tile_queue_stride(int64_t bytes);
 
 // The GEMM stage's workspace: the tile kernels' queue (without one their tiles
 // are dealt statically); the other kernels need none.
@@ -268,7 +269,7 @@ int launch_int4_gemm(const void* A, int a_dtype, int64_t M, int64_t K, const int
                   reinterpret_cast<uintptr_t>(workspace) % 4 == 0
               ? static_cast<int*>(workspace)
               : nullptr,
-          queue_cleared, stream);
+          tile_queue_stride(workspace_bytes), queue_cleared, stream);
     }
     case Int4Kernel::kRs:
       return launch_int4_rs(A, a_dtype == XK_DT_FP32, M, K, packed, scale, E, N, numel, top_k,

@@ -67,8 +67,9 @@ struct PrefillArgs {
   float* out;              // [numel, N]
   int K, N, numel, top_k, num_experts;
   int glog;                // log2(group size / 32)
-  int* queue;              // [kXcds] tiles taken from each XCD's range (zero at launch), or null
+  int* queue;              // tiles taken from each XCD's range (zero at launch), or null
   int a_bytes;             // bytes of A
+  int queue_stride;        // ints from one XCD's counter to the next
 };
 
 // GBIG: groups of 64 or 128 (chunk 4 s + q's scale is scale[(4 s + q) >> glog]);
@@ -163,7 +164,7 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& p) {
           const int x = (xcd + k) % kXcds;
           const int nx = xcd_tiles(x);
           if (nx > 0) {
-            const int n = atomicAdd(&p.queue[x], 1);
+            const int n = atomicAdd(&p.queue[x * p.queue_stride], 1);
             if (n < nx) tt = xcd_tile(x, n);
           }
         }
@@ -381,7 +382,7 @@ int4_prefill_gemm_g(PrefillArgs p) {
 
 int device_cu_count();
 
-int launch_clear_queue(int* q, int n, hipStream_t stream);
+int launch_clear_queue(int* q, int n, int stride, hipStream_t stream);
 
 // Shapes the tile kernel takes: bf16 activations, groups of 32, 64 or 128, K a
 // multiple of two steps, N a multiple of the column tile, at most kPMaxExperts
@@ -396,17 +397,17 @@ bool int4_prefill_ok(int a_dtype, int group_size, int64_t M, int64_t K, int64_t 
 int launch_int4_prefill(const void* A, int64_t K, const int32_t* packed, const uint16_t* scale,
                         int64_t E, int64_t N, int64_t numel, int64_t top_k, int group_size,
                         const int32_t* sorted_ids, const int32_t* offsets, float* slot_out,
-                        int* queue, bool queue_cleared, hipStream_t stream) {
+                        int* queue, int queue_stride, bool queue_cleared, hipStream_t stream) {
   XK_REQUIRE(reinterpret_cast<uintptr_t>(A) % 16 == 0 && reinterpret_cast<uintptr_t>(packed) % 16 == 0,
              "int4 prefill: A and packed must be 16-byte aligned");
   const int64_t a_bytes = numel / std::max<int64_t>(top_k, 1) * K * 2;
   XK_REQUIRE(a_bytes < (int64_t(1) << 31) && N * K / 2 < (int64_t(1) << 31),
              "int4 prefill: A and one expert's weights must each be below 2^31 bytes");
   if (queue != nullptr && !queue_cleared)
-    if (int rc = launch_clear_queue(queue, kXcds, stream)) return rc;
+    if (int rc = launch_clear_queue(queue, kXcds, queue_stride, stream)) return rc;
   PrefillArgs a{static_cast<const uint16_t*>(A), reinterpret_cast<const uint32_t*>(packed), scale,
                 sorted_ids, offsets, slot_out, int(K), int(N), int(numel), int(top_k), int(E),
-                group_size == 128 ? 2 : group_size == 64 ? 1 : 0, queue, int(a_bytes)};
+                group_size == 128 ? 2 : group_size == 64 ? 1 : 0, queue, int(a_bytes), queue_stride};
   // one workgroup per CU, a multiple of the XCD count
   const int cus = device_cu_count();
   const int grid = std::max(kXcds, cus / kXcds * kXcds);
