@@ -297,19 +297,24 @@ def _mxfp4_tiles(M, E, hidden, ispp, top_k, f32=False, experts=0):
 
 
 @pytest.mark.parametrize("M,E,hidden,ispp,k,f32,experts,want", [
-    # the tile kernel took up to twice the passes' time at these (measured)
+    # few rows and a short contraction: passes (measured)
     (1, 256, 4096, 512, 6, True, 0, (False, False)),
-    (16, 64, 2048, 1408, 8, True, 0, (False, False)),
-    (60, 32, 2880, 2880, 4, True, 0, (False, False)),
-    (120, 32, 2848, 2912, 4, False, 0, (False, False)),
     (16, 1024, 2048, 512, 8, False, 0, (False, False)),
     (107, 32, 4096, 512, 6, False, 256, (False, False)),
-    (512, 32, 4096, 512, 6, False, 256, (False, False)),
-    # and less from here on
+    (448, 64, 256, 256, 4, False, 0, (False, False)),
+    (200, 32, 512, 512, 4, False, 0, (False, False)),
+    # a contraction that is not a multiple of 512
+    (120, 32, 2848, 2912, 4, False, 0, (False, False)),
+    (60, 32, 2880, 2880, 4, True, 0, (False, False)),
+    (1024, 64, 256, 2048, 4, False, 0, (True, True)),
+    (200, 32, 2848, 2912, 4, False, 0, (True, True)),
+    # tiles
+    (16, 64, 2048, 1408, 8, True, 0, (True, False)),
+    (600, 1, 512, 512, 1, False, 0, (True, True)),
+    (512, 32, 4096, 512, 6, False, 256, (True, True)),
     (128, 256, 4096, 512, 6, True, 0, (True, False)),
     (400, 64, 2048, 1408, 8, True, 0, (True, True)),
-    (400, 32, 2848, 2912, 4, False, 0, (True, True)),
-    (2048, 32, 4096, 512, 6, False, 256, (True, False)),
+    (2048, 32, 4096, 512, 6, False, 256, (True, True)),
     (4096, 256, 4096, 512, 6, False, 0, (True, True)),
     (64, 128, 7168, 2048, 8, True, 0, (True, True)),
 ])

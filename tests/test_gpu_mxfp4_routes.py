@@ -1,5 +1,5 @@
 """fused_moe_mxfp4 off its stream path: 32-row passes, 128-row tiles, and one for
-each projection, as the rows per expert and the number of tiles choose. fp32
+each projection, as the rows per expert, the contraction and the number of tiles choose. fp32
 activations, sizes that are odd multiples of 32, more than 512 experts, scales
 at odd addresses and expert maps, each at few and at many rows, against the
 oracle; every scratch byte starts as a NaN pattern, so a row that nothing wrote
@@ -11,6 +11,7 @@ import torch
 
 from oracle.torch_ref import moe_mxfp4_ref
 from tests._helpers import softmax_weights, uniform_topk, zipf_topk
+from tests.test_capi import _mxfp4_tiles
 from xkernels_amd import Backend, MoeMxfp4Workspace, fused_moe_mxfp4, make_mxfp4_moe_weights
 
 pytestmark = pytest.mark.gpu
@@ -51,14 +52,17 @@ def _check(M, E, hidden, ispp, k, dev, dtype=torch.bfloat16, experts=0, routing=
     assert float((got - want).norm()) <= 2e-3 * float(want.norm()) + 1e-6
 
 
-@pytest.mark.parametrize("M,E,hidden,ispp,k,routing", [
-    (1, 8, 512, 512, 2, "uniform"),    # few rows: passes
-    (33, 2, 256, 160, 2, "uniform"),   # 33 rows an expert: two passes, tiles for gate/up
-    (40, 4, 544, 96, 1, "zipf"),
-    (300, 8, 2048, 256, 4, "zipf"),    # tiles for gate/up, passes for down
-    (600, 8, 2048, 1408, 4, "zipf"),   # tiles for both
+@pytest.mark.parametrize("M,E,hidden,ispp,k,routing,tiles", [  # tiles: of gate/up, of down; else passes
+    (1, 8, 512, 512, 2, "uniform", (False, False)),
+    (33, 2, 256, 160, 2, "uniform", (False, False)),  # 33 rows an expert: two passes
+    (40, 4, 544, 96, 1, "zipf", (False, False)),
+    (300, 8, 2048, 256, 4, "zipf", (True, True)),
+    (300, 8, 2048, 64, 4, "zipf", (True, False)),
+    (600, 8, 32, 1536, 4, "zipf", (False, True)),
+    (600, 8, 2048, 1408, 4, "zipf", (True, True)),
 ])
-def test_fp32_activations(M, E, hidden, ispp, k, routing, dev):
+def test_fp32_activations(M, E, hidden, ispp, k, routing, tiles, dev):
+    assert _mxfp4_tiles(M, E, hidden, ispp, k, True) == tiles
     _check(M, E, hidden, ispp, k, dev, dtype=torch.float32, routing=routing)
 
 
@@ -68,8 +72,9 @@ def test_odd_multiples_of_32(hidden, ispp, M, E, k, routing, dev):
     _check(M, E, hidden, ispp, k, dev, routing=routing)
 
 
-@pytest.mark.parametrize("M", [7, 300])
-def test_more_than_512_experts(M, dev):
+@pytest.mark.parametrize("M,tiles", [(7, False), (300, False), (6000, True)])
+def test_more_than_512_experts(M, tiles, dev):
+    assert _mxfp4_tiles(M, 600, 256, 128, 8) == (tiles, tiles)
     _check(M, 600, 256, 128, 8, dev)
 
 
@@ -81,7 +86,9 @@ def test_scales_at_odd_addresses(hidden, ispp, shift, M, dev):
 
 @pytest.mark.parametrize("M,E,experts,hidden,ispp,k", [
     (60, 8, 64, 256, 192, 6),      # few local rows of many slots: passes
-    (300, 4, 16, 256, 96, 4),      # 75 local rows an expert: tiles and passes
+    (300, 4, 16, 256, 96, 4),      # 75 local rows an expert, three passes
+    (300, 4, 16, 1024, 96, 4),     # tiles for gate/up, passes for down
+    (400, 4, 16, 96, 1024, 4),     # the other way round
     (400, 4, 16, 2048, 1024, 4),   # tiles for both
     (64, 2, 64, 544, 160, 8),
     (200, 4, 8, 512, 512, 3),      # top_k with no fixed-size combine

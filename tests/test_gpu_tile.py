@@ -14,6 +14,7 @@ import torch
 
 from oracle.torch_ref import moe_mxfp4_ref
 from tests._helpers import softmax_weights
+from tests.test_capi import _mxfp4_tiles
 from tests.test_gpu_int4_exact import _bounded_check, _device_inputs, _gemm_rows
 from xkernels_amd import Backend, _lib, fused_moe_mxfp4, make_mxfp4_moe_weights
 
@@ -115,3 +116,46 @@ def test_mxfp4_tile_edges(hidden, ispp, dtype, dev):
     # bf16 roundings of the gate/up sums, the activation and the down sums that
     # fall on other sides of a tie: 2^-9 relative each on a small share of terms
     assert float((got - want).norm() / want.norm()) < 2e-3
+
+
+# 128-row blocks and tails of every height, at rows enough for tiles of any K
+LONG_ROWS = [770, 801, 897, 577]
+
+
+@pytest.mark.parametrize("hidden,ispp", [(32, 32), (96, 32), (160, 96), (2080, 160), (544, 1376)])
+def test_mxfp4_tiles_of_short_contractions(hidden, ispp, dev):
+    """K below, between and past the multiples of a chunk (128) and of a scale
+    block (512), in both projections."""
+    E, M = len(LONG_ROWS), sum(LONG_ROWS)
+    print(f"mxfp4 tiles hidden={hidden} ispp={ispp}", flush=True)
+    assert _mxfp4_tiles(M, E, hidden, ispp, 1) == (True, True)
+    wts = make_mxfp4_moe_weights(E, hidden, ispp, with_bias=True, device="cpu", seed=hidden, scale_lo=115,
+                                 scale_hi=122)
+    A = torch.randn(M, hidden, generator=torch.Generator().manual_seed(1)).to(torch.bfloat16)
+    ids, w = _row_ids(LONG_ROWS, ispp), softmax_weights(M, 1, 3) * 0.7
+    keys = ("w13", "w13_scale", "w2", "w2_scale")
+    got = fused_moe_mxfp4(A.to(dev), *(wts[k].to(dev) for k in keys), ids.to(dev), w.to(dev),
+                          b13=wts["b13"].to(dev), b2=wts["b2"].to(dev), backend=Backend.HIP).float().cpu()
+    want = moe_mxfp4_ref(A, *(wts[k] for k in keys), ids, w, b13=wts["b13"], b2=wts["b2"]).float()
+    assert torch.isfinite(got).all()
+    # the bound of test_mxfp4_tile_edges
+    assert float((got - want).norm() / want.norm()) < 2e-3
+
+
+@pytest.mark.parametrize("hidden,ispp,tiles", [(60064, 32, (True, False)), (32, 60064, (False, True))])
+def test_mxfp4_tile_of_one_token(hidden, ispp, tiles, dev):
+    """One activation row and a partial last chunk, at a contraction long enough
+    that one token takes the tile kernel: loads past K and of pad rows land zeros
+    though their scalar offset passes the end of A."""
+    assert _mxfp4_tiles(1, 1, hidden, ispp, 1, False) == tiles
+    print(f"mxfp4 one token in tiles hidden={hidden} ispp={ispp}", flush=True)
+    wts = make_mxfp4_moe_weights(1, hidden, ispp, with_bias=True, device="cpu", seed=3, scale_lo=112, scale_hi=118)
+    A = torch.randn(1, hidden, generator=torch.Generator().manual_seed(3)).to(torch.bfloat16)
+    ids, w = torch.zeros(1, 1, dtype=torch.int32), torch.full((1, 1), 0.7)
+    keys = ("w13", "w13_scale", "w2", "w2_scale")
+    # fp32 activations: no stream kernel
+    got = fused_moe_mxfp4(A.float().to(dev), *(wts[k].to(dev) for k in keys), ids.to(dev), w.to(dev),
+                          b13=wts["b13"].to(dev), b2=wts["b2"].to(dev), backend=Backend.HIP).cpu()
+    want = moe_mxfp4_ref(A.float(), *(wts[k] for k in keys), ids, w, b13=wts["b13"], b2=wts["b2"])
+    # the bound of test_mxfp4_one_token
+    assert float((got - want).norm() / want.norm()) < 4e-3

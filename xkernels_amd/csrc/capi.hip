@@ -497,33 +497,41 @@ struct Mxfp4Plan {
 };
 
 // The kernel of each projection off the stream path: 128-row tiles (true) or
-// 32-row passes (mxfp4_stream_gemm). A pass costs each workgroup its weights
-// once per 32 rows; a tile costs a fixed start and end (a ticket, the first
-// chunk's loads, the stores) and needs many tiles on the 512 places, which rows,
-// experts, columns and the length of the contraction K all bring. Measured per
-// call, the tile's time less the passes':
-//   gate/up, bf16: E = 32, hidden 2848, ispp 2912: +35 us at 15 rows per expert,
-//     +9 at 25, -28 at 32; 32 of 256 experts, hidden 4096, ispp 512: +22 at 12,
-//     -1 at 24, -18 at 32; E = 1024, hidden 2048, ispp 512: +9 at 256 slots, -23
-//     at 512, -49 at 1,024; E = 600, hidden 7168, ispp 2048: -84 at 64 slots.
-//   gate/up, fp32 (the passes read twice the bytes): E = 64, hidden 2048, ispp
-//     1408: +6 at 2 rows per expert, -14 at 16; E = 32, hidden = ispp = 2880: +5
-//     at 2, +17 at 8, -1 at 15; E = 64, hidden 4096, ispp 2048: +2 at 16 slots,
-//     -27 at 32.
-//   down: E = 256, hidden 4096, ispp 512: +27 at 3 rows, +15 at 24, -9 at 32, -37
-//     at 48; 32 of 256 experts +28 at 48, +11 at 96; E = 64, hidden 2048, ispp
-//     1408: +15 at 30, -6 at 50; E = 32, hidden = ispp = 2880: +29 at 15, +1 at
-//     25, -38 at 50; E = 128, hidden 7168, ispp 2048: -35 at 1 row.
+// 32-row passes (mxfp4_stream_gemm). A pass costs each workgroup its weights and
+// their dequant once per 32 rows; a tile costs a few us of start and end (a
+// ticket, the first chunk's loads, the stores), which the length of the
+// contraction K times the rows must earn back, and sooner where there are tiles
+// for all 512 places. Measured per call with cold weights, the tile's time less
+// the passes' (MXFP4, bf16):
+//   few tiles: E = 16, K = 512, gate/up: +2 at 20 rows per expert, 0 at 30, -4 at
+//     64; K = 1024: 0 at 8, -2 at 20, -7 at 24; K = 4096: -10 at 8, -45 at 30;
+//   many: E = 256, K = 512, gate/up: +1 at 12, -3 at 24, -15 at 48; down -15 at 8;
+//   K not a multiple of 512 (a scale load per group): E = 16, K = 256: +3 at 48
+//     rows, 0 at 96, -7 at 160; E = 256, K = 256, gate/up of 1,024 tiles: +5 at 24,
+//     -3 at 36, -14 at 64; E = 32, hidden = ispp = 2880, gate/up: +7 at 12, +3 at
+//     20, -25 at 25; down: +18 at 8, +15 at 20, -8 at 25.
+// Passes read fp32 activations in full, twice the bytes of a row. Batches of less
+// than a row per expert are decided by the columns and K (gate/up tile less
+// passes: E = 600, hidden 7168, ispp 2048, 64 slots: -84 us; down: E = 128,
+// hidden 7168, ispp 2048, 1 row: -35).
 }  // namespace
 namespace xk {
+namespace {
+bool tile_rows_pay(int64_t local, int64_t E, int64_t K, int64_t col_tiles, double pass_cost) {
+  const bool many = std::min(local, E) * col_tiles * cdiv(cdiv(local, E), 128) >= 512;
+  const int64_t from = K % 512 == 0 ? (many ? 6000 : 20000) : K >= 2048 ? 60000 : many ? 10000 : 24000;
+  return pass_cost * double(local) * double(K) >= double(from * E);
+}
+}  // namespace
 bool mxfp4_tile_gate_up(int64_t local, int64_t E, int64_t hidden, int64_t ispp, bool f32) {
-  return local >= (f32 ? 14 : 28) * E ||
-         std::min(local, E) * cdiv(ispp, 128) * hidden * hidden >= (int64_t(1) << 33);
+  const int64_t col_tiles = cdiv(ispp, 128);
+  return tile_rows_pay(local, E, hidden, col_tiles, f32 ? 2.0 : 1.0) ||
+         (hidden % 512 == 0 && std::min(local, E) * col_tiles * hidden * hidden >= (int64_t(1) << 33));
 }
 bool mxfp4_tile_down(int64_t local, int64_t E, int64_t hidden, int64_t ispp) {
   const int64_t col_tiles = cdiv(hidden, 256);
-  return (local >= 28 * E && local * col_tiles * ispp >= 28000000) ||
-         std::min(local, E) * col_tiles * ispp * ispp >= (int64_t(1) << 32);
+  return tile_rows_pay(local, E, ispp, col_tiles, 1.0) ||
+         (ispp % 512 == 0 && std::min(local, E) * col_tiles * ispp * ispp >= (int64_t(1) << 32));
 }
 }  // namespace xk
 namespace {
