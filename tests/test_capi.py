@@ -342,12 +342,14 @@ def test_mxfp4_workspace_serves_smaller_batches():
 
 
 @pytest.mark.parametrize("M,E,N,K,k,experts,want", [
-    (1, 64, 64, 7168, 8, 0, True), (1, 48, 4096, 7168, 8, 0, True), (6, 48, 4096, 7168, 8, 0, True),
-    (6, 48, 7168, 2048, 8, 0, True), (6, 48, 7168, 2048, 8, 384, True), (1, 64, 512, 2048, 8, 0, True),
+    (1, 48, 4096, 7168, 8, 0, True), (3, 48, 4096, 7168, 8, 0, True), (3, 48, 7168, 2048, 8, 0, True),
+    (6, 48, 7168, 2048, 8, 384, True), (1, 64, 512, 2048, 8, 0, True), (2, 256, 4096, 2048, 8, 0, True),
     (6, 8, 1024, 2048, 2, 0, True), (6, 4, 256, 7168, 4, 0, True),
     # few columns and many experts: the stream kernel takes a quarter to half the time
     (6, 64, 16, 7168, 8, 0, False), (3, 64, 256, 7168, 8, 0, False), (6, 64, 1024, 7168, 8, 0, False),
     (6, 64, 512, 2048, 8, 0, False), (3, 64, 512, 2048, 8, 0, False), (6, 16, 2048, 4096, 4, 0, False), (2, 64, 256, 14336, 8, 0, False), (6, 64, 4096, 10240, 8, 0, False),
+    # a few more workgroups than CUs, and rows that leave a CU one of them
+    (3, 48, 5120, 7168, 8, 0, False), (6, 48, 5120, 7168, 8, 0, False), (4, 8, 256, 14336, 2, 0, False),
 ])
 def test_int4_one_launch_kernel_choice(M, E, N, K, k, experts, want):
     lib, i64, ptr = _lib.load(), ctypes.c_int64, ctypes.c_void_p(256)
@@ -358,10 +360,13 @@ def test_int4_one_launch_kernel_choice(M, E, N, K, k, experts, want):
 
 @pytest.mark.parametrize("M,E,hidden,ispp,k,want", [
     (1, 256, 4096, 512, 6, True), (6, 256, 4096, 512, 6, True), (3, 64, 4096, 1024, 8, True),
-    (5, 256, 7168, 512, 8, True), (2, 64, 7168, 2048, 8, True),
+    (5, 256, 7168, 512, 8, True), (2, 64, 7168, 2048, 8, True), (6, 8, 7168, 512, 1, True),
+    (1, 8, 7168, 8192, 2, True), (1, 8, 1024, 6144, 2, True),
+    # a long ispp for few experts: most waves of the down projection idle
+    (1, 8, 4096, 14336, 2, False), (2, 8, 1024, 8192, 2, False), (1, 8, 1024, 10240, 1, False),
     # rows that leave a CU one workgroup: the stream kernel is faster
     (6, 256, 7168, 512, 8, False), (4, 64, 4096, 1024, 8, False), (4, 32, 2048, 2048, 4, False),
-    (7, 256, 4096, 512, 6, False), (1, 256, 4096, 544, 6, False), (5, 64, 512, 512, 13, False),
+    (7, 256, 4096, 512, 6, False), (1, 256, 4096, 544, 6, False), (6, 256, 1024, 512, 8, False), (5, 64, 512, 512, 13, False),
 ])
 def test_mxfp4_small_kernels_choice(M, E, hidden, ispp, k, want):
     lib, i64, ptr = _lib.load(), ctypes.c_int64, ctypes.c_void_p(256)

@@ -18,10 +18,10 @@
 //   * its waves split (expert, 512-k unit) pairs evenly, each with the next
 //     unit's 16-byte loads in flight while one is contracted.
 // Per call, stream path -> here: INT4 at N = 4096, K = 7168, 1 / 2 / 4 / 8 tokens
-// 46 -> 31, 67 -> 57, 93 -> 86, 124 -> 123 us (fewer columns: small_int4_faster); N = 7168, K = 2048, 1 / 4 / 8
-// tokens 25.5 -> 19, 51 -> 48, 67 -> 68 us; MXFP4, 1 / 4 / 8 tokens 28.8 -> 19.1,
-// 39 -> 28, 53.5 -> 53 us. From 8 tokens on the experts' weights hide the
-// latencies either way.
+// 46 -> 31, 67 -> 57, 93 -> 86, 124 -> 123 us (other sizes: small_int4_faster); N =
+// 7168, K = 2048, 1 / 4 / 8 tokens 25.5 -> 19, 51 -> 48, 67 -> 68 us; MXFP4, 1 / 4 /
+// 8 tokens 28.8 -> 19.1, 39 -> 28, 53.5 -> 53 us. From 8 tokens on the experts'
+// weights hide the latencies either way.
 #include <algorithm>
 #include <cmath>
 
@@ -364,28 +364,36 @@ small_mxfp4_down(SmallArgs p) {
   }
 }
 
-constexpr int64_t kSmallLds = 140 * 1024;  // beside the static arrays (12 KiB)
+constexpr int64_t kSmallLds = 140 * 1024;  // beside the static arrays
+constexpr int64_t kStaticLds = 12 * 1024, kTwoWorkgroupLds = 80 * 1024;
 int64_t row_lds(int64_t rows, int64_t K) { return rows * (K + kRowPad) * 2; }
 
 bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
 
 }  // namespace
 
-// A workgroup of small_int4 walks the weights of 16 columns for every expert X of
-// the batch, about 2 + X (K + 1000) / 3000 us whatever N is; the stream kernel
-// splits experts x columns over all CUs, about 14 + K / 1300 + X N K / 10^7 us. So
-// it runs for few experts, or for so many columns that the weights take longer
-// than their latencies (up to a size where the stream kernel reads them a little
-// better). E = 64, top_k 8, stream vs here: K = 7168, N = 1024: 1 token 27 vs 25
-// us, 3 tokens 33 vs 55, 6 tokens 44 vs 97; N = 64: 1 token 24 vs 24, 6 tokens 25
-// vs 92; K = 2048, N = 512: 1 token 19 vs 13, 3 tokens 19 vs 23, 6 tokens 20 vs
-// 34; N = 4096: E = 48, K = 7168, 6 tokens 107 vs 101, K = 10240 161 vs 167.
+// Whether small_int4 is expected to be faster than the stream kernel, from fits to
+// both kernels' times with cold weights (2,130 sizes: X = 1 to 48 experts, N = 256
+// to 14336, K = 512 to 14336; mean error 8 %; where the choice is wrong it costs 4
+// us or less but for a few sizes). A workgroup walks the weights of 16 columns for
+// every expert X of the batch, so beyond the bytes its time grows with X K per
+// workgroup of a CU, more where the rows in the LDS leave a CU one workgroup of
+// eight waves; the stream kernel splits experts x columns over all CUs. Stream vs
+// here: N = 4096, K = 7168, E = 48, top_k 8: 1 token 44 vs 33 us, 3 tokens 69 vs
+// 64, 6 tokens 114 vs 115; N = 7168, K = 2048: 3 tokens 41 vs 37, 6 tokens 61 vs
+// 64; N = 5120, K = 7168: 3 tokens 81 vs 108, 6 tokens 142 vs 229; E = 8, top_k 2,
+// N = 256, K = 14336, 4 tokens 24 vs 42; E = 256, top_k 8, N = 4096, K = 2048, 2
+// tokens 30 vs 21.
 bool small_int4_faster(int64_t M, int64_t top_k, int64_t E, int64_t routed, int64_t N, int64_t K) {
   // local experts that `M` tokens' slots are expected to reach
   const double miss = 1.0 - double(std::min(top_k, routed)) / double(routed);
   const double experts = double(E) * (1.0 - std::pow(miss, double(M)));
-  return experts * double(K + 1000) <= 38000.0 + 3.85 * double(K) ||
-         (N * K >= 3296 * (K + 1000) && experts * double(K) <= 300000.0);
+  const double k1 = double(K) / 1e3, all = experts * double(N) * double(K) / 1e7;
+  const int64_t cus = device_cu_count(), per_cu = cdiv(N / 16, cus);
+  const bool alone = per_cu > 1 && row_lds(M, K) + kStaticLds > kTwoWorkgroupLds;
+  const double here = 5.0 + 0.09 * experts + k1 * (experts * double(per_cu) * (alone ? 0.46 : 0.3) + 0.085 * double(M)) + 0.3 * all;
+  const double stream = 10.5 + 0.1 * experts + k1 + 0.89 * all + 1.5e-6 * double(M * top_k) * double(N);
+  return here < stream;
 }
 
 // Batches the one-launch INT4 kernel takes: bf16 activations, groups of 32, at
@@ -418,19 +426,28 @@ int launch_small_int4(const uint16_t* A, int64_t M, int64_t K, const int32_t* pa
 }
 
 // MXFP4: the same, for hidden and ispp multiples of 512, with rows in the LDS that
-// leave room for two workgroups a CU; the down projection loads a row per slot in
-// every workgroup, which costs it more from 3 tokens on. Stream vs here: E = 256, hidden 7168, ispp
-// 512, top_k 8, 5 tokens (70 KiB) 64 vs 62 us, 6 tokens (84 KiB) 73 vs 95; E = 64,
-// hidden 4096, ispp 1024, top_k 8, 3 tokens (down 48 KiB) 43 vs 42, 4 tokens (64.5
-// KiB) 50 vs 53, 6 tokens (97 KiB) 62 vs 73; hidden 7168, ispp 2048, 2 tokens
-// (64.3 KiB) 84 vs 79.
-constexpr int64_t kSmallGateUpLds = 72 * 1024, kSmallDownLds = 64 * 1024;
+// leave room for two workgroups a CU where there are so many, and a down projection
+// that its waves can share: a wave takes whole experts, so few experts of a long
+// ispp leave most waves idle (sooner where few columns leave the CUs idle too), and
+// every workgroup loads a row per slot, which costs it more from 3 tokens on.
+// Stream vs here, cold weights: E = 256, hidden 7168, ispp 512, top_k 8, 5 tokens
+// (70 KiB) 64 vs 62 us, 6 tokens (84 KiB) 73 vs 95, but E = 8, top_k 1 (up to 256
+// workgroups) 27 vs 16; E = 64, hidden 4096, ispp 1024, top_k 8, 3 tokens (down 48
+// KiB) 43 vs 42, 4 tokens (64.5 KiB) 50 vs 53; E = 8, hidden 1024, top_k 2: ispp
+// 8192, 2 tokens 29 vs 35, ispp 14336, 1 token 33 vs 46; hidden 7168, ispp 8192, 1
+// token 59 vs 51; E = 256, hidden 1024, ispp 512, top_k 8, 6 tokens 32 vs 34.
+constexpr int64_t kSmallGateUpLds = 72 * 1024, kSmallDownLds = 64 * 1024, kSmallLoneLds = 128 * 1024;
 bool small_mxfp4_ok(int a_dtype, int64_t M, int64_t top_k, int64_t E, int64_t hidden, int64_t ispp, const void* A,
                     const void* w13, const void* w13_scale, const void* w2, const void* w2_scale) {
-  return a_dtype == XK_DT_BF16 && M >= 1 && M <= kMaxTokens && M * top_k <= kSlots && hidden % kUnitK == 0 &&
-         ispp % kUnitK == 0 && hidden < (1 << 24) && ispp < (1 << 24) && E <= 1024 &&
-         row_lds(M, hidden) <= kSmallGateUpLds && row_lds(M * top_k, ispp) <= (M <= 2 ? kSmallGateUpLds : kSmallDownLds) && aligned16(A) &&
-         aligned16(w13) && aligned16(w13_scale) && aligned16(w2) && aligned16(w2_scale);
+  if (a_dtype != XK_DT_BF16 || M < 1 || M > kMaxTokens || M * top_k > kSlots || hidden % kUnitK != 0 ||
+      ispp % kUnitK != 0 || hidden >= (1 << 24) || ispp >= (1 << 24) || E > 1024)
+    return false;
+  const int64_t numel = M * top_k, gate_up = row_lds(M, hidden), down = row_lds(numel, ispp);
+  const bool few = ispp / 16 * std::min(E, numel) <= 2 * device_cu_count();
+  return gate_up <= (few ? kSmallLoneLds : kSmallGateUpLds) && down <= (M <= 2 ? kSmallGateUpLds : kSmallDownLds) &&
+         ispp * cdiv(numel, 8) <= (hidden >= 4096 ? 8192 : 7168) &&
+         (hidden > 1024 || numel <= 8 || numel * ispp < 24576) && aligned16(A) && aligned16(w13) &&
+         aligned16(w13_scale) && aligned16(w2) && aligned16(w2_scale);
 }
 
 int launch_small_mxfp4(const uint16_t* A, int64_t M, int64_t hidden, const uint8_t* w13, const uint8_t* s13,
