@@ -377,8 +377,8 @@ def test_mxfp4_small_kernels_choice(M, E, hidden, ispp, k, want):
 
 @pytest.mark.parametrize("rows,E,N,K,want", [
     # stream (1) or tile (2) at sizes that are not multiples of 256, rows per expert
-    (33, 48, 2880, 2880, 1), (50, 48, 2880, 2880, 2), (64, 16, 2880, 2880, 1), (100, 16, 2880, 2880, 2),
-    (100, 16, 2880, 1024, 1), (400, 16, 2880, 1024, 2), (42, 8, 2880, 512, 1), (400, 8, 2880, 512, 1),
+    (33, 48, 2880, 2880, 1), (50, 48, 2880, 2880, 2), (50, 8, 2880, 2880, 1), (100, 16, 2880, 2880, 2),
+    (50, 64, 1440, 1440, 2), (1200, 16, 720, 544, 2), (42, 8, 2880, 512, 1), (1200, 1, 1440, 2880, 1),
     (1600, 8, 2880, 512, 2), (400, 8, 128, 512, 1), (512, 8, 16, 512, 1), (42, 48, 7184, 2048, 2),
 ])
 def test_int4_kernel_of_padded_sizes(rows, E, N, K, want):
@@ -387,14 +387,16 @@ def test_int4_kernel_of_padded_sizes(rows, E, N, K, want):
     assert _lib.query("xk_moe_int4_kernel", rows * E, 8, E, N, K, _lib.XK_DT_BF16, 32, 0, 8 * E) == want
 
 
-@pytest.mark.parametrize("rows,E,N,want", [
+@pytest.mark.parametrize("rows,E,N,K,want", [
     # 256-row (True) or 128-row tiles, rows per expert
-    (18, 48, 4096, False), (100, 48, 4096, False), (133, 48, 4096, True), (256, 48, 4096, False),
-    (683, 48, 4096, True), (25, 48, 7168, False), (180, 48, 7168, True),
-    (18, 16, 2048, True), (100, 16, 2048, True), (400, 16, 2048, True), (18, 64, 512, True), (400, 64, 512, True),
-    (42, 48, 2048, True), (18, 8, 1024, False), (400, 8, 1024, False),
+    (18, 48, 4096, 7168, False), (100, 48, 4096, 7168, False), (128, 48, 4096, 7168, False),
+    (180, 48, 4096, 7168, True), (256, 48, 4096, 7168, False), (683, 48, 4096, 7168, False),
+    (25, 48, 7168, 2048, False), (180, 48, 7168, 2048, True), (180, 16, 2048, 4096, False),
+    (100, 16, 2048, 4096, False), (400, 64, 512, 2048, False), (42, 48, 2048, 2048, False),
+    (400, 8, 1024, 4096, False), (100, 48, 2048, 512, False), (128, 48, 2048, 512, True),
+    (320, 48, 2048, 512, True), (500, 8, 4096, 512, True), (500, 8, 1024, 512, False),
 ])
-def test_int4_tile_height(rows, E, N, want):
-    tall = _lib.load()["_ZN2xk15int4_tall_tilesElll"]
+def test_int4_tile_height(rows, E, N, K, want):
+    tall = _lib.load()["_ZN2xk15int4_tall_tilesEllll"]
     tall.restype = ctypes.c_bool
-    assert tall(*(ctypes.c_int64(x) for x in (rows * E, E, N))) == want
+    assert tall(*(ctypes.c_int64(x) for x in (rows * E, E, N, K))) == want

@@ -109,48 +109,41 @@ int launch_int4_prefill(const void* A, int64_t K, const int32_t* packed, const u
 // Routed rows per expert (on average) from which the tile kernels replace the
 // weight-streaming kernel, which streams every expert's weights once per
 // 16-row pass. Measured per fused call, stream vs tile (moe_tile), uniform
-// routing: E = 48, N = 4096, K = 7168, top_k = 8: 172 vs 217 us at 10.7 rows
-// per expert, 191 vs 218 at 13.3, 244 vs 221 at 16.7, 311 vs 226 at 21.7, 483
-// vs 256 at 42. One line for all shapes, drawn at this one: N = 7168, K = 2048
-// crosses at 25 rows (134 vs 161 at 18, 166 vs 167 at 25, 192 vs 190 at 33), and
-// experts whose tiles do not fill the chip later still (E = 16, N = K = 4096: 56
-// vs 81 at 18, 92 vs 85 at 42).
+// routing: E = 48, N = 4096, K = 7168, top_k = 8: 170 vs 201 us at 12 rows per
+// expert, 248 vs 205 at 17, 321 vs 215 at 24, 559 vs 249 at 48. One line for all
+// shapes, drawn at this one: N = 7168, K = 2048 crosses at 20 rows (124 vs 136 at
+// 17, 162 vs 144 at 24), and few experts later (E = 16, N = K = 4096: 53 vs 54 at
+// 17; N = 2048, K = 4096: 42 vs 49 at 24, 49 vs 50 at 32).
 constexpr int64_t kPrefillRowsPerExpert = 17;
 // K or N not a multiple of 256: the tile pads both, the stream kernel little. It
 // runs from 40 rows per expert on where the stream kernel's work (local slots x N
-// x K at about 120 million products a us) takes longer than a few rounds of tiles:
-// about 55 us and K / 60 us a round of the 512 places. Per fused call, stream vs
-// tile: E = 48, N = K = 2880: 127 vs 149 us at 33 rows, 153 vs 154 at 42, 172 vs
-// 160 at 50; E = 16, N = K = 2880: 79 vs 102 at 64, 110 vs 91 at 100; E = 16, N =
-// 2880, K = 1024: 50 vs 66 at 100, 78 vs 78 at 180; E = 8, N = 2880, K = 512: 19 vs
-// 50 at 42, 61 vs 74 at 400, 103 vs 99 at 800; E = 8, N = 128, K = 512: 28 vs 37 at
-// 400.
+// x K at about 100 million products a us) takes longer than a few rounds of tiles:
+// about 15 us and K / 80 us a round of the 512 places. Per fused call, stream vs
+// tile: E = 48, N = K = 2880: 146 vs 159 us at 40 rows; E = 64, N = K = 1440: 87
+// vs 62 at 50; E = 16, N = 720, K = 544: 134 vs 56 at 1,200; E = 8, N = K = 2880:
+// 50 vs 53 at 70; E = 1, N = 1440, K = 2880: 54 vs 64 at 1,200.
 constexpr int64_t kPaddedTileRowsPerExpert = 40;
 bool int4_padded_tile(int64_t rows, int64_t E, int64_t N, int64_t K) {
   const int64_t tiles = E * cdiv(N, 256) * cdiv(cdiv(rows, E), 128);
-  return rows >= kPaddedTileRowsPerExpert * E && double(rows) * N * K >= 120e6 * (55.0 + K * cdiv(tiles, 512) / 60.0);
+  return rows >= kPaddedTileRowsPerExpert * E && double(rows) * N * K >= 100e6 * (15.0 + K * cdiv(tiles, 512) / 80.0);
 }
 
 // The 256-row tile kernel (int4_prefill_gemm, one 8-wave workgroup a CU) in place
-// of the 128-row one (moe_tile, two 4-wave workgroups), by routed rows per expert.
-// It runs
-//   * where most experts fill one 256-row tile but need two of 128 rows, and in
-//     batches of several 256-row tiles per expert, where its one dequant per 256
-//     rows saves about 1 %. N = 4096, K = 7168, E = 48, per fused call 256- vs
-//     128-row: 405 vs 343 us at 100 rows, 492 vs 517 at 133, 549 vs 610 at 167,
-//     655 vs 663 at 217, 821 vs 770 at 256, 1,043 vs 965 at 333, 1,388 vs 1,347 at
-//     500, 1,858 vs 1,877 at 683; N = 7168, K = 2048: 268 vs 252 at 100, 295 vs 302
-//     at 128, 361 vs 402 at 180, 505 vs 496 at 256, 740 vs 734 at 400;
-//   * where the tiles do not fill the chip, so that a tile has a CU to itself and
-//     eight waves finish it before four: K = 4096, N = 2048, E = 16 (128 tiles): 64
-//     vs 80 us at 18 rows, 68 vs 85 at 50, 143 vs 158 at 400; K = 2048, N = 512, E =
-//     64: 50 vs 70 at 18, 95 vs 117 at 400; N = 2048, E = 48 (384 tiles): 69 vs 73
-//     at 18, 74 vs 81 at 42, 97 vs 92 at 80; but N = 1024, E = 8 (32 tiles): 48 vs
-//     37 at 18; N = 1024, K = 4096, E = 8 (64 tiles): 124 vs 104 at 400.
-bool int4_tall_tiles(int64_t rows, int64_t E, int64_t N) {
-  if ((rows >= 120 * E && rows < 224 * E) || rows >= 600 * E) return true;
+// of the 128-row one (moe_tile, two 4-wave workgroups). It runs where most experts
+// fill one 256-row tile but need two of 128 rows and there are tiles enough for
+// all CUs, and at a short K with a round of 256-row tiles or more, where a tile is
+// mostly its start and end and half as many are better. Per fused call, 256- vs
+// 128-row, by rows per expert: N = 4096, K = 7168, E = 48: 399 vs 330 us at 100,
+// 455 vs 448 at 128, 559 vs 595 at 180, 709 vs 672 at 240, 1,344 vs 1,296 at 500,
+// 1,843 vs 1,798 at 680; N = 7168, K = 2048: 292 vs 277 at 128, 367 vs 391 at 180,
+// 455 vs 435 at 240, 1,147 vs 1,136 at 680; too few tiles: N = 2048, K = 4096, E =
+// 16: 119 vs 80 at 180; K = 512, N = 2048, E = 48: 53 vs 43 at 100, 57 vs 65 at
+// 128, 93 vs 104 at 320, 130 vs 136 at 500; K = 512, N = 4096, E = 8 (256 tiles):
+// 63 vs 71 at 500; K = 1024, N = 1024, E = 128: 78 vs 87 (K = 512) at 180.
+bool int4_tall_tiles(int64_t rows, int64_t E, int64_t N, int64_t K) {
+  if (rows < 120 * E) return false;
   const int64_t tiles = E * cdiv(N, 256) * cdiv(cdiv(rows, E), 256);
-  return rows < 120 * E ? tiles >= 64 && tiles <= 384 : tiles >= 128 && tiles <= 512;
+  return (K <= 1024 && tiles >= 256) || (rows >= 140 * E && rows < 224 * E && tiles >= 384);
 }
 
 int64_t tile_queue_bytes();
@@ -259,7 +252,7 @@ int launch_int4_gemm(const void* A, int a_dtype, int64_t M, int64_t K, const int
     case Int4Kernel::kTile: {
       // groups of 64 and 128 stay on the 256-row kernel (one scale load per
       // group and chunk in moe_tile: 120 tokens 264 vs 274 us, 1,400 Zipf 735 vs 790)
-      const bool tall = (group_size != 32 || int4_tall_tiles(int4_local_slots(numel, E, ep_global), E, N)) &&
+      const bool tall = (group_size != 32 || int4_tall_tiles(int4_local_slots(numel, E, ep_global), E, N, K)) &&
                         int4_prefill_ok(a_dtype, group_size, M, K, N, E);
       // the tile queue lives in the workspace; without one the tiles are
       // dealt statically
