@@ -400,3 +400,13 @@ def test_int4_tile_height(rows, E, N, K, want):
     tall = _lib.load()["_ZN2xk15int4_tall_tilesEllll"]
     tall.restype = ctypes.c_bool
     assert tall(*(ctypes.c_int64(x) for x in (rows * E, E, N, K))) == want
+
+
+@pytest.mark.parametrize("E,k,M", [
+    # rows from which the router's 16 lanes a row take less time than 64 (measured)
+    (128, 8, 0), (8, 1, 1500), (129, 1, 3000), (256, 4, 1300), (256, 8, 1024), (256, 16, 16), (257, 8, 3200), (512, 1, 6000),
+])
+def test_router_lanes_per_row(E, k, M):
+    rows = _lib.load()["_ZN2xk11rows16_fromEii"]
+    rows.restype = ctypes.c_int64
+    assert rows(E, k) == M

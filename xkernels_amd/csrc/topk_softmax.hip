@@ -3,7 +3,7 @@
 // renormalisation of the selected weights (contract of the reference's
 // src/xkernels/ops/moe/topk_softmax.py:33-95 and its Op Spec).
 //
-// Rows of up to 512 experts with k up to 16 take 16 lanes each
+// Rows of up to 512 experts with k up to 16 take 16 lanes each in larger batches
 // (topk_softmax_rows16 below). Otherwise one wave64 owns one row at a time. Lane
 // l holds experts l, l+64, l+128, ...
 // (every load instruction of the wave reads one contiguous run of logits), so a
@@ -142,7 +142,7 @@ topk_softmax_rows(const T* __restrict__ logits, int64_t M, int E, int k, int ren
   }
 }
 
-// Rows of up to 512 experts, k up to 16: 16 lanes a row, four rows a wave. The
+// Rows of up to 512 experts, k up to 16 (rows16_from): 16 lanes a row, four rows a wave. The
 // selection rounds are VALU work (six instructions per key and round, the
 // cross-lane steps beside), and a row's 16 lanes reduce with four DPP moves in
 // place of six LDS permutes: the four rows of a wave cost about what one row
@@ -328,12 +328,33 @@ hipError_t launch_rows16(const void* logits, int64_t M, int E, int k, int renorm
   return hipGetLastError();
 }
 
+// Rows from which 16 lanes a row are faster than 64. A row's selection is four
+// times as long on 16 lanes, which only batches that fill the chip hide, and
+// beyond 128 experts it no longer pays for itself in cheaper cross-lane steps.
+// Kernel times in us, 64 vs 16 lanes, bf16 (fp32 lies within 0.5 us):
+//   E = 128: k = 1: 3.1 vs 3.0 at 1,024 rows; k = 8: 4.6 vs 4.2 at 1, 5.5 vs 4.5
+//     at 1,024; E = 16, k = 1: 3.0 vs 3.1 at 1,024, 3.1 vs 3.1 at 1,500;
+//   E = 256: k = 1: 3.7 vs 3.8 at 2,048, 4.0 vs 3.9 at 3,000; k = 2: 3.9 vs 4.1 at
+//     1,024, 4.2 vs 4.2 at 2,048; k = 8: 5.3 vs 6.0 at 1, 6.3 vs 6.1 at 1,024, 9.4
+//     vs 6.3 at 4,096; k = 16: 8.0 vs 9.1 at 1, 9.2 vs 8.7 at 64;
+//   E = 384: k = 1: 5.2 vs 5.3 at 4,096, 12.3 vs 10.5 at 16,384; k = 8: 7.5 vs 9.3
+//     at 1,024, 9.4 vs 9.3 at 3,000, 10.8 vs 9.5 at 4,096; k = 16: 9.6 vs 14.8 at
+//     1, 12.7 vs 14.0 at 2,048, 14.9 vs 14.1 at 3,000.
+}  // namespace
+int64_t rows16_from(int E, int k) {
+  if (E <= 128) return k < 4 ? 1500 : 0;
+  if (E <= 256) return k < 2 ? 3000 : k < 4 ? 2048 : k < 8 ? 1300 : k == 8 ? 1024 : 16;
+  return k < 4 ? 6000 : k < 8 ? 4096 : 3200;
+}
+namespace {
+
 template <typename T>
 hipError_t launch_typed(const void* logits, int64_t M, int E, int k, int renorm, float* w,
                         int32_t* ids, hipStream_t stream) {
   // a launch takes fewer than 2^32 threads (16 a row here; the kernels below
   // loop over the rows)
-  if (k <= 16 && E <= 512 && cdiv(M, kTsThreads / 16) * kTsThreads < (int64_t(1) << 32)) {
+  if (k <= 16 && E <= 512 && M >= rows16_from(E, k) &&
+      cdiv(M, kTsThreads / 16) * kTsThreads < (int64_t(1) << 32)) {
     if (E <= 128) return launch_rows16<T, 1>(logits, M, E, k, renorm, w, ids, stream);
     if (E <= 256) return launch_rows16<T, 2>(logits, M, E, k, renorm, w, ids, stream);
     return launch_rows16<T, 4>(logits, M, E, k, renorm, w, ids, stream);
