@@ -1,13 +1,14 @@
-"""The prefill-regime INT4 tile kernel (MFMA tiles of 256 routed rows x 256
-columns) against the oracle and against the decode stream kernel.
+"""The prefill-regime INT4 tile kernels against the oracle and against the decode
+stream kernel: tiles of 128 routed rows x 256 columns, which the cases below take
+by their rows per expert, and of 256 x 256, which test_256_row_kernel forces.
 
-Both kernels dequantise to the reference's bf16-rounded weights, so their fp32
+The kernels dequantise to the reference's bf16-rounded weights, so their fp32
 per-slot rows differ only by fp32 summation order (checked at 1e-4 relative);
 the fused outputs meet the op spec's bf16 tolerance against the oracle. Cases
 cover skewed (Zipf) routing with partial and empty row blocks, experts with no
 tokens, more tiles than workgroups, expert parallelism and the unweighted sum,
-and fixed per-expert row counts that give every tile height (256, 192, 128 and
-64 rows) and every tile order class.
+and fixed per-expert row counts that give the 256-row kernel every tile height
+(256, 192, 128 and 64 rows) and every tile order class.
 """
 from __future__ import annotations
 
@@ -108,11 +109,11 @@ CASES = [  # M, E, N, K, top_k, routing
 
 
 @pytest.mark.parametrize("M,E,N,K,top_k,routing", CASES)
-def test_tile_kernel_rows_match_stream_kernel(M, E, N, K, top_k, routing, dev):
+def test_tile_kernel_rows_match_stream_kernel(M, E, N, K, top_k, routing, dev, force=_lib._XK_INT4_TEST_FORCE_TILE):
     print(f"tile vs stream M={M} E={E} N={N} K={K} k={top_k} {routing}", flush=True)
     ids = _ids(M, top_k, E, routing, M)
     A, packed, scale, ids, _ = _inputs(M, E, N, K, ids, seed=M + 3)
-    tile = _slot_rows(A, packed, scale, ids, _lib._XK_INT4_TEST_FORCE_TILE)
+    tile = _slot_rows(A, packed, scale, ids, force)
     stream = _slot_rows(A, packed, scale, ids, _lib._XK_INT4_TEST_FORCE_STREAM)
     torch.cuda.synchronize()
     assert not torch.isnan(tile).any(), "a routed slot row was not written"
@@ -120,7 +121,7 @@ def test_tile_kernel_rows_match_stream_kernel(M, E, N, K, top_k, routing, dev):
 
 
 @pytest.mark.parametrize("M,E,N,K,top_k,routing", CASES)
-def test_tile_queue_equals_static_deal(M, E, N, K, top_k, routing, dev):
+def test_tile_queue_equals_static_deal(M, E, N, K, top_k, routing, dev, force=_lib._XK_INT4_TEST_FORCE_TILE):
     """The tile queue (workgroups take tiles atomically, then the other XCDs'
     ranges) computes every tile exactly once: its rows equal the static deal's
     bit for bit, from a buffer of NaNs, over two calls with one workspace."""
@@ -130,28 +131,28 @@ def test_tile_queue_equals_static_deal(M, E, N, K, top_k, routing, dev):
     need = _lib.query("xk_moe_int4_gemm_workspace_bytes", M, K)
     assert need > 0
     gws = torch.randint(0, 256, (need,), dtype=torch.uint8, device=dev)  # the queue is cleared per call
-    static = _slot_rows(A, packed, scale, ids, _lib._XK_INT4_TEST_FORCE_TILE)
+    static = _slot_rows(A, packed, scale, ids, force)
     for _ in range(2):
-        queued = _slot_rows(A, packed, scale, ids, _lib._XK_INT4_TEST_FORCE_TILE, gws)
+        queued = _slot_rows(A, packed, scale, ids, force, gws)
         torch.cuda.synchronize()
         assert not torch.isnan(queued).any(), "a routed slot row was not written"
         assert torch.equal(queued, static)
 
 
 @pytest.mark.parametrize("M,E,N,K,top_k,routing", CASES)
-def test_tile_kernel_matches_oracle(M, E, N, K, top_k, routing, dev):
+def test_tile_kernel_matches_oracle(M, E, N, K, top_k, routing, dev, force=_lib._XK_INT4_TEST_FORCE_TILE):
     print(f"tile vs oracle M={M} E={E} N={N} K={K} k={top_k} {routing}", flush=True)
     ids = _ids(M, top_k, E, routing, M + 1)
     A, packed, scale, ids, w = _inputs(M, E, N, K, ids, seed=M + 5)
-    got = _fused(A, packed, scale, ids, w, _lib._XK_INT4_TEST_FORCE_TILE)
+    got = _fused(A, packed, scale, ids, w, force)
     assert_close(got, moe_w4a16_ref(A, packed, scale, ids, w), 2e-2, 2e-2, "tile fused")
 
 
-def test_tile_kernel_unweighted_and_expert_parallel(dev):
+def test_tile_kernel_unweighted_and_expert_parallel(dev, force=_lib._XK_INT4_TEST_FORCE_TILE):
     M, E, N, K, k = 512, 16, 512, 1024, 4
     ids = zipf_topk(M, k, E, 1.1, 77)
     A, packed, scale, ids, w = _inputs(M, E, N, K, ids, seed=78)
-    got = _fused(A, packed, scale, ids, w, _lib._XK_INT4_TEST_FORCE_TILE, mul=0)
+    got = _fused(A, packed, scale, ids, w, force, mul=0)
     assert_close(got, moe_w4a16_ref(A, packed, scale, ids, w, mul_routed_weight=False), 2e-2, 2e-2,
                  "tile unweighted")
     dense = moe_w4a16_ref(A, packed, scale, ids, w).float()
@@ -160,9 +161,22 @@ def test_tile_kernel_unweighted_and_expert_parallel(dev):
         emap = torch.full((E,), -1, dtype=torch.int32, device="cuda")
         emap[r * 8:(r + 1) * 8] = torch.arange(8, dtype=torch.int32, device="cuda")
         lp, ls = packed[r * 8:(r + 1) * 8].contiguous(), scale[r * 8:(r + 1) * 8].contiguous()
-        part = _fused(A, lp, ls, ids, w, _lib._XK_INT4_TEST_FORCE_TILE, emap=emap)
+        part = _fused(A, lp, ls, ids, w, force, emap=emap)
         total += part.float()
     assert_close(total, dense, 3e-2, 3e-2, "tile EP partials")
+
+
+@pytest.mark.parametrize("M,E,N,K,top_k,routing", CASES)
+def test_256_row_kernel(M, E, N, K, top_k, routing, dev):
+    """The same cases on tiles of 256 rows (K a multiple of 256, N too)."""
+    tall = _lib._XK_INT4_TEST_FORCE_TILE | _lib._XK_INT4_TEST_TALL
+    test_tile_kernel_rows_match_stream_kernel(M, E, N, K, top_k, routing, dev, tall)
+    test_tile_queue_equals_static_deal(M, E, N, K, top_k, routing, dev, tall)
+    test_tile_kernel_matches_oracle(M, E, N, K, top_k, routing, dev, tall)
+
+
+def test_256_row_kernel_unweighted_and_expert_parallel(dev):
+    test_tile_kernel_unweighted_and_expert_parallel(dev, _lib._XK_INT4_TEST_FORCE_TILE | _lib._XK_INT4_TEST_TALL)
 
 
 def test_default_choice_uses_tile_kernel_at_prefill_sizes(dev):

@@ -26,6 +26,7 @@ XK_DT_NONE = -1
 # pick the tile or the stream kernel where the shapes allow both.
 _XK_INT4_TEST_FORCE_TILE = 1 << 8
 _XK_INT4_TEST_FORCE_STREAM = 1 << 9
+_XK_INT4_TEST_TALL = 1 << 11
 
 _p = ctypes.c_void_p
 _i32 = ctypes.c_int32

@@ -284,7 +284,7 @@ int xk_moe_int4_w4a16_gemm(const void* A, int32_t a_dtype, int64_t M, int64_t K,
                            float* slot_out, int32_t flags, void* workspace,
                            int64_t workspace_bytes, hipStream_t stream) {
   clear_error();
-  XK_REQUIRE((flags & ~(XK_INT4_TEST_FORCE_TILE | XK_INT4_TEST_FORCE_STREAM)) == 0,
+  XK_REQUIRE((flags & ~XK_INT4_TEST_BITS) == 0,
              "int4: unknown flags 0x%x (pass 0)", flags);
   return launch_int4_gemm(A, a_dtype, M, K, packed, scale, E, N, group_size, topk_ids, top_k,
                           expert_map, num_global_experts, sorted_token_ids, expert_offsets,
@@ -315,7 +315,7 @@ int xk_moe_int4_w4a16(const void* A, int32_t a_dtype, int64_t M, int64_t K,
   XK_REQUIRE(out != nullptr || M == 0, "int4: null out");
   XK_REQUIRE(M == 0 || (A && packed && scale && topk_ids), "int4: null input pointer");
   XK_REQUIRE(!mul_routed_weight || topk_w || M == 0, "int4: null topk_w");
-  XK_REQUIRE((flags & ~(XK_INT4_TEST_FORCE_TILE | XK_INT4_TEST_FORCE_STREAM)) == 0,
+  XK_REQUIRE((flags & ~XK_INT4_TEST_BITS) == 0,
              "int4: unknown flags 0x%x (pass 0)", flags);
   if (M == 0) return XK_OK;
   const int64_t need = xk_moe_int4_w4a16_workspace_bytes(M, top_k, E, N, K);
@@ -414,7 +414,7 @@ int xk_moe_int4_w4a16_noalloc(const void* A, int32_t a_dtype, int64_t M, int64_t
   XK_REQUIRE(M >= 0 && top_k >= 1 && E >= 1 && N >= 1 && K >= 1,
              "int4 noalloc: bad sizes M=%lld top_k=%lld E=%lld N=%lld K=%lld", (long long)M,
              (long long)top_k, (long long)E, (long long)N, (long long)K);
-  XK_REQUIRE((flags & ~(XK_INT4_TEST_FORCE_TILE | XK_INT4_TEST_FORCE_STREAM)) == 0,
+  XK_REQUIRE((flags & ~XK_INT4_TEST_BITS) == 0,
              "int4 noalloc: unknown flags 0x%x (pass 0)", flags);
   if (M == 0) return XK_OK;
   const int64_t need = xk_moe_int4_w4a16_workspace_bytes(M, top_k, E, N, K);

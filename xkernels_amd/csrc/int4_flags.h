@@ -8,6 +8,9 @@
 
 #define XK_INT4_TEST_FORCE_TILE (1 << 8)
 #define XK_INT4_TEST_FORCE_STREAM (1 << 9)
+// with FORCE_TILE: the 256-row tile kernel where it takes the shape
+#define XK_INT4_TEST_TALL (1 << 11)
+#define XK_INT4_TEST_BITS (XK_INT4_TEST_FORCE_TILE | XK_INT4_TEST_FORCE_STREAM | XK_INT4_TEST_TALL)
 // Set by the fused call (and the query of its kernel) alone, never accepted from
 // a caller: K or N not a multiple of 256 may take the tile kernel. The stage
 // entry keeps such shapes on the stream kernel, whose calls may come without

@@ -252,7 +252,7 @@ int launch_int4_gemm(const void* A, int a_dtype, int64_t M, int64_t K, const int
     case Int4Kernel::kTile: {
       // groups of 64 and 128 stay on the 256-row kernel (one scale load per
       // group and chunk in moe_tile: 120 tokens 264 vs 274 us, 1,400 Zipf 735 vs 790)
-      const bool tall = (group_size != 32 || int4_tall_tiles(int4_local_slots(numel, E, ep_global), E, N, K)) &&
+      const bool tall = ((flags & XK_INT4_TEST_TALL) || group_size != 32 || int4_tall_tiles(int4_local_slots(numel, E, ep_global), E, N, K)) &&
                         int4_prefill_ok(a_dtype, group_size, M, K, N, E);
       // the tile queue lives in the workspace; without one the tiles are
       // dealt statically
