@@ -390,10 +390,10 @@ def test_int4_kernel_of_padded_sizes(rows, E, N, K, want):
 @pytest.mark.parametrize("rows,E,N,K,want", [
     # 256-row (True) or 128-row tiles, rows per expert
     (18, 48, 4096, 7168, False), (100, 48, 4096, 7168, False), (128, 48, 4096, 7168, False),
-    (180, 48, 4096, 7168, True), (256, 48, 4096, 7168, False), (683, 48, 4096, 7168, False),
+    (180, 48, 4096, 7168, True), (256, 48, 4096, 7168, False), (500, 48, 4096, 7168, False), (683, 48, 4096, 7168, True),
     (25, 48, 7168, 2048, False), (180, 48, 7168, 2048, True), (180, 16, 2048, 4096, False),
     (100, 16, 2048, 4096, False), (400, 64, 512, 2048, False), (42, 48, 2048, 2048, False),
-    (400, 8, 1024, 4096, False), (100, 48, 2048, 512, False), (128, 48, 2048, 512, True),
+    (400, 8, 1024, 4096, False), (680, 4, 1024, 4096, False), (100, 48, 2048, 512, False), (128, 48, 2048, 512, True),
     (320, 48, 2048, 512, True), (500, 8, 4096, 512, True), (500, 8, 1024, 512, False),
 ])
 def test_int4_tile_height(rows, E, N, K, want):

@@ -129,21 +129,24 @@ bool int4_padded_tile(int64_t rows, int64_t E, int64_t N, int64_t K) {
 }
 
 // The 256-row tile kernel (int4_prefill_gemm, one 8-wave workgroup a CU) in place
-// of the 128-row one (moe_tile, two 4-wave workgroups). It runs where most experts
-// fill one 256-row tile but need two of 128 rows and there are tiles enough for
-// all CUs, and at a short K with a round of 256-row tiles or more, where a tile is
-// mostly its start and end and half as many are better. Per fused call, 256- vs
-// 128-row, by rows per expert: N = 4096, K = 7168, E = 48: 399 vs 330 us at 100,
-// 455 vs 448 at 128, 559 vs 595 at 180, 709 vs 672 at 240, 1,344 vs 1,296 at 500,
-// 1,843 vs 1,798 at 680; N = 7168, K = 2048: 292 vs 277 at 128, 367 vs 391 at 180,
-// 455 vs 435 at 240, 1,147 vs 1,136 at 680; too few tiles: N = 2048, K = 4096, E =
-// 16: 119 vs 80 at 180; K = 512, N = 2048, E = 48: 53 vs 43 at 100, 57 vs 65 at
-// 128, 93 vs 104 at 320, 130 vs 136 at 500; K = 512, N = 4096, E = 8 (256 tiles):
-// 63 vs 71 at 500; K = 1024, N = 1024, E = 128: 78 vs 87 (K = 512) at 180.
+// of the 128-row one (moe_tile, two 4-wave workgroups). It runs, with tiles enough
+// for all CUs, where most experts fill one 256-row tile but need two of 128 rows,
+// and in the largest batches, where both draw the card's power limit and its one
+// dequant per 256 rows saves up to 1 %; and at a short K with a round of 256-row
+// tiles or more, where a tile is mostly its start and end and half as many are
+// better. Per fused call, 256- vs 128-row, by rows per expert: N = 4096, K = 7168,
+// E = 48: 399 vs 330 us at 100, 455 vs 448 at 128, 559 vs 595 at 180, 709 vs 672 at
+// 240, 1,222 vs 1,228 at 400, Zipf 1,191 vs 1,167; N = 7168, K = 2048: 292 vs 277
+// at 128, 367 vs 391 at 180, 455 vs 435 at 240; from 680 rows on 0.5 % more to 1.3 %
+// less at four shapes (calls back to back; E = 48, 4,096 tokens, Zipf 1,848 vs
+// 1,875); too few tiles: N = 2048, K = 4096, E = 16: 119 vs 80 at 180; K = 512, N =
+// 2048, E = 48: 53 vs 43 at 100, 57 vs 65 at 128, 93 vs 104 at 320, 130 vs 136 at
+// 500; K = 512, N = 4096, E = 8 (256 tiles): 63 vs 71 at 500.
 bool int4_tall_tiles(int64_t rows, int64_t E, int64_t N, int64_t K) {
   if (rows < 120 * E) return false;
   const int64_t tiles = E * cdiv(N, 256) * cdiv(cdiv(rows, E), 256);
-  return (K <= 1024 && tiles >= 256) || (rows >= 140 * E && rows < 224 * E && tiles >= 384);
+  if (K <= 1024 && tiles >= 256) return true;
+  return tiles >= 384 && ((rows >= 140 * E && rows < 224 * E) || rows >= 600 * E);
 }
 
 int64_t tile_queue_bytes();
@@ -252,7 +255,8 @@ int launch_int4_gemm(const void* A, int a_dtype, int64_t M, int64_t K, const int
     case Int4Kernel::kTile: {
       // groups of 64 and 128 stay on the 256-row kernel (one scale load per
       // group and chunk in moe_tile: 120 tokens 264 vs 274 us, 1,400 Zipf 735 vs 790)
-      const bool tall = ((flags & XK_INT4_TEST_TALL) || group_size != 32 || int4_tall_tiles(int4_local_slots(numel, E, ep_global), E, N, K)) &&
+      const bool tall = ((flags & XK_INT4_TEST_TALL) || group_size != 32 ||
+                         int4_tall_tiles(int4_local_slots(numel, E, ep_global), E, N, K)) &&
                         int4_prefill_ok(a_dtype, group_size, M, K, N, E);
       // the tile queue lives in the workspace; without one the tiles are
       // dealt statically
