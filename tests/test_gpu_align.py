@@ -99,7 +99,7 @@ def test_cpu_tensor_is_rejected():
         moe_align_block_size(torch.zeros((2, 2), dtype=torch.int32), 4, 4, backend=Backend.HIP)
 
 
-@pytest.mark.parametrize("numel,E", [(2048, 48), (2049, 48), (3072, 8), (4097, 384), (8192, 512), (8193, 1024)])
+@pytest.mark.parametrize("numel,E", [(2048, 48), (2049, 48), (3072, 8), (3073, 8), (2049, 31), (2049, 32), (4097, 384), (8192, 512), (8193, 1024)])
 def test_grid_path_edges(numel, E, dev):
     """Slot counts around the one-workgroup path's limit and whole and partial
     1024-slot chunks, with dropped ids in every chunk; the fused calls' queue

@@ -171,7 +171,6 @@ align_single_wg(const int32_t* __restrict__ ids, int64_t numel, int num_experts,
                 int32_t* __restrict__ expert_ids, int32_t* __restrict__ num_post,
                 int32_t* __restrict__ expert_offsets, int* __restrict__ clear, int nclear, int clear_stride) {
   extern __shared__ int lds[];
-  if (static_cast<int>(threadIdx.x) < nclear) clear[threadIdx.x * clear_stride] = 0;
   const int nw = blockDim.x >> 6;
   int* cnt = lds;                               // [E]   histogram, then cursor
   int* off = cnt + num_experts;                 // [E+1] padded prefix
@@ -190,6 +189,7 @@ align_single_wg(const int32_t* __restrict__ ids, int64_t numel, int num_experts,
   __syncthreads();
   chunk_stable_scatter(ids, 0, numel, emap, num_global, num_experts, cnt, wavecnt, tot,
                        sorted_ids);
+  if (static_cast<int>(threadIdx.x) < nclear) clear[threadIdx.x * clear_stride] = 0;
 }
 
 // Grid phase 1: histogram of chunk b into chunk_cnt[b][0..E).
@@ -329,15 +329,16 @@ align_place(const int32_t* __restrict__ ids, int64_t numel, int nchunks,
 }
 
 // One workgroup takes rounds of 1024 slots with five barriers each; the grid
-// path's two launches cost about two rounds more (one workgroup: 8.4 us at 2,000
-// slots, 20.6 us at 6,216). Without the grid path's workspace one workgroup
-// takes up to 8192 slots.
-constexpr int64_t kSingleWgBestSlots = 2048;
+// path's two launches cost about two rounds more, and three with few experts, whose
+// rounds are shorter (one workgroup vs grid: E = 64, 2,048 slots 7.6 us, 2,049 9.0
+// vs 7.8; E = 8, 3,000 slots 8.4 vs 9.3, 4,096 10.0 vs 9.4). Without the grid
+// path's workspace one workgroup takes up to 8192 slots.
+int64_t single_wg_best_slots(int num_experts) { return num_experts < 32 ? 3072 : 2048; }
 constexpr int64_t kSingleWgMaxSlots = 8192;
 constexpr int kSingleWgMaxExperts = 512;
 
 bool use_single_wg(int64_t numel, int num_experts, bool workspace) {
-  return numel <= (workspace ? kSingleWgBestSlots : kSingleWgMaxSlots) && num_experts <= kSingleWgMaxExperts;
+  return numel <= (workspace ? single_wg_best_slots(num_experts) : kSingleWgMaxSlots) && num_experts <= kSingleWgMaxExperts;
 }
 
 }  // namespace
