@@ -332,8 +332,9 @@ int xk_moe_int4_w4a16(const void* A, int32_t a_dtype, int64_t M, int64_t K,
   // through buffer offsets) runs as the fewest even token chunks that they
   // take: a token's output depends only on its own slots (each slot
   // row is a fixed-order K sum, the combine sums a token's slots in slot
-  // order), so the chunks write what one call would, bit for bit, with the
-  // MFMA kernels instead of the scalar one. Each chunk lays out its smaller
+  // order). Chunks of one size take one kernel; calls over another split of the
+  // batch write the same bits where their sizes choose that kernel too, else the
+  // same sums in another fp32 order. Each chunk lays out its smaller
   // workspace at the start of this one; the stream orders them.
   const int fused = flags | XK_INT4_FUSED;
   if (flags == 0 && int4_kernel_code(M, top_k, E, N, K, a_dtype, group_size, fused, 0) == 0) {

@@ -146,7 +146,8 @@ bool int4_tall_tiles(int64_t rows, int64_t E, int64_t N, int64_t K) {
   if (rows < 120 * E) return false;
   const int64_t tiles = E * cdiv(N, 256) * cdiv(cdiv(rows, E), 256);
   if (K <= 1024 && tiles >= 256) return true;
-  return tiles >= 384 && ((rows >= 140 * E && rows < 224 * E) || rows >= 600 * E);
+  if (rows >= 600 * E) return E * cdiv(N, 256) >= 128;  // not by rows: parts of a batch take one kernel
+  return rows >= 140 * E && rows < 224 * E && tiles >= 384;
 }
 
 int64_t tile_queue_bytes();
