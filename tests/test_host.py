@@ -42,6 +42,19 @@ def test_dispatch_explicit_env_and_auto(fake_kernel, monkeypatch):
     assert _dispatch.select_backend(fake_kernel) is Backend.REFERENCE
 
 
+@pytest.mark.parametrize("vendor", ["amd", "nvidia", "none"])
+@pytest.mark.parametrize("have", [("reference",), ("hip",), ("triton", "reference"), ("hip", "reference"),
+                                  ("cuda", "triton"), ("reference", "triton", "hip", "cuda")])
+def test_dispatch_runs_what_select_backend_names(fake_kernel, monkeypatch, vendor, have):
+    for b in have:
+        _dispatch.register(fake_kernel, Backend(b))(lambda b=b: b)
+    monkeypatch.delenv("XKERNELS_BACKEND", raising=False)
+    monkeypatch.setattr(_dispatch, "detect_vendor", lambda: vendor)
+    assert _dispatch.dispatch(fake_kernel) == _dispatch.select_backend(fake_kernel).value
+    monkeypatch.setenv("XKERNELS_BACKEND", have[-1])
+    assert _dispatch.dispatch(fake_kernel) == _dispatch.select_backend(fake_kernel).value == have[-1]
+
+
 def test_dispatch_unregistered_backend_raises(fake_kernel, monkeypatch):
     _dispatch.register(fake_kernel, Backend.REFERENCE)(lambda: 0)
     with pytest.raises(KeyError, match="not registered"):

@@ -171,8 +171,12 @@ def select_backend(kernel_name: str, backend="auto") -> Backend:
         if want not in e.impls:
             raise _missing(kernel_name, want, e)
         return want
-    order = _PREFERENCE.get(detect_vendor(), (Backend.REFERENCE,))
-    for b in order:
+    return _automatic(e)
+
+
+def _automatic(e: _Entry) -> Backend:
+    """The backend of ``backend="auto"`` with no environment override."""
+    for b in _PREFERENCE.get(detect_vendor(), (Backend.REFERENCE,)):
         if b in e.impls:
             return b
     return next(iter(e.impls))
@@ -201,18 +205,11 @@ def _warn_if_passed_over(kernel: str, chosen: Backend, args, kwargs) -> None:
 def dispatch(kernel_name: str, *args, backend="auto", **kwargs):
     """Runs ``kernel_name`` on the selected backend."""
     if backend == "auto" and not os.environ.get("XKERNELS_BACKEND", "").strip():
-        # an automatic choice, resolved here without a second look at the
-        # environment (select_backend's last rule; it also raises the errors)
+        # select_backend without its second look at the environment (it raises the errors)
         e = _TABLE.get(kernel_name)
-        if e is not None and e.impls:
-            for b in _PREFERENCE.get(detect_vendor(), (Backend.REFERENCE,)):
-                fn = e.impls.get(b)
-                if fn is not None:
-                    if b is Backend.REFERENCE:
-                        _warn_if_passed_over(kernel_name, b, args, kwargs)
-                    return fn(*args, **kwargs)
-        chosen = select_backend(kernel_name, backend)
-        _warn_if_passed_over(kernel_name, chosen, args, kwargs)
+        chosen = _automatic(e) if e is not None and e.impls else select_backend(kernel_name)
+        if chosen is Backend.REFERENCE:
+            _warn_if_passed_over(kernel_name, chosen, args, kwargs)
     else:
         chosen = select_backend(kernel_name, backend)
     return _TABLE[kernel_name].impls[chosen](*args, **kwargs)
