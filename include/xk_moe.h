@@ -109,7 +109,9 @@ int xk_moe_sum_reduce(const void* y, int32_t y_dtype, int64_t M, int64_t top_k,
  *   out[m] = sum_j [w[m,j]] * (A[m] @ W[e_j]^T),  e_j = topk_ids[m, j]
  * A [M, K] bf16|fp32, out [M, N] in A's dtype, topk_w fp32 [M, top_k].
  * expert_map (nullable) selects this rank's experts; the result is then the
- * rank's partial output. Runs align -> grouped GEMM -> weighted combine.
+ * rank's partial output. Batches of up to 6 tokens and 64 slots may run one
+ * kernel; else decode batches run the grouped GEMM, which routes the slots
+ * itself, and the weighted combine, larger ones the align before them.
  * ------------------------------------------------------------------------- */
 int64_t xk_moe_int4_w4a16_workspace_bytes(int64_t M, int64_t top_k, int64_t E,
                                           int64_t N, int64_t K);
@@ -137,7 +139,9 @@ int xk_moe_int4_w4a16(const void* A, int32_t a_dtype, int64_t M, int64_t K,
  * arguments without the workspace; the scratch is a fixed device array of
  * xk_moe_int4_w4a16_noalloc_max_bytes() bytes (64 MiB) inside the library,
  * one per GPU, held until the process ends. A call whose
- * xk_moe_int4_w4a16_workspace_bytes(...) exceeds it fails with XK_ERR_INVALID.
+ * xk_moe_int4_w4a16_workspace_bytes(...) exceeds it fails with XK_ERR_INVALID;
+ * of that size the align's scratch does not count (up to 16 KiB) for batches of
+ * up to 8192 slots on up to 512 experts.
  * Every call on one GPU uses the same array: calls that overlap on a GPU (two
  * streams, two host threads) race; calls ordered on one stream do not. */
 int64_t xk_moe_int4_w4a16_noalloc_max_bytes(void);
@@ -168,12 +172,14 @@ int xk_moe_int4_w4a16_noalloc(const void* A, int32_t a_dtype, int64_t M, int64_t
  * call does this and skips the align). Used by benchmarks to time the GEMM
  * alone. */
 int32_t xk_moe_int4_block_size(int64_t M, int64_t top_k, int64_t E);
-/* Which grouped-GEMM kernel a fused call with these shapes runs: 0 the scalar
+/* Which grouped-GEMM kernel a fused call with these shapes runs where it does not
+ * run the one kernel of the smallest batches (up to 6 tokens; its choice also
+ * depends on the pointers' alignment): 0 the scalar
  * kernel (shapes the MFMA kernels do not take, including activations or one
  * expert's packed weights of 2^31 bytes or more; the fused call runs a batch
  * whose activations reach 2^31 bytes as token chunks, each with the choice for
  * its own M), 1 the decode weight-streaming
- * kernel, 2 the prefill MFMA tile kernel. num_global_experts: the expert map's
+ * kernel, 2 a prefill MFMA tile kernel (of 128 or 256 rows). num_global_experts: the expert map's
  * size for an expert-parallel call with a workspace of
  * xk_moe_int4_w4a16_ep_workspace_bytes, else 0. No counterpart in the
  * reference (its Triton launcher has no such query); for tests and tooling. */
