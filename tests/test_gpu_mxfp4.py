@@ -39,12 +39,13 @@ def _ref(A, wts, ids, w, **kw):
 
 
 # bf16 A and fewer than 20 routed rows per expert on average: both projections
-# run the stream kernel (fp32 partial planes, SwiGLU and combine kernels);
-# other shapes the per-stage kernels. Hidden 384 / ispp 640: K not a multiple
+# run the stream kernel (fp32 partial planes, SwiGLU and combine kernels) or,
+# up to 6 tokens, the small-batch kernels; other shapes each projection on
+# 32-row passes or tiles. Hidden 384 / ispp 640: K not a multiple
 # of 256 (but of 128), the last 256-k line zero-padded.
 # 600 x 8 = 4800 routed slots on 256 experts: more than the stream kernel
 # routes itself, so the align outputs feed it; 200 x 8 on 64 experts (25 rows
-# per expert) runs the per-stage kernels.
+# per expert) runs off the stream path.
 STREAM_SHAPES = [(4, 8, 256, 256, 2), (1, 16, 512, 256, 6), (48, 32, 512, 512, 6),
                  (33, 4, 256, 512, 2), (100, 64, 256, 256, 8), (600, 256, 256, 256, 8),
                  (200, 64, 256, 256, 8), (8, 16, 384, 640, 4), (8, 384, 256, 256, 6)]
@@ -98,8 +99,8 @@ def test_fp32_activations(dev):
 
 @pytest.mark.parametrize("ispp", [64, 256])
 def test_full_scale_range_and_special_codes(ispp, dev):
-    """Scale bytes across [110, 135) plus 0xFF (reads as 0) and 0 (2^-127) in both
-    the 256-k stream kernel and the generic kernel (ispp 64)."""
+    """Scale bytes across [110, 135) plus 0xFF (reads as 0) and 0 (2^-127) in the
+    stream kernel with 16-byte and (ispp 64) with 2-byte scale loads."""
     A, wts, ids, w = _case(6, 4, 256, ispp, 2, seed=6, scale_lo=110, scale_hi=135)
     wts["w2_scale"][0, :3, 0] = 255
     wts["w13_scale"][1, 5, 2] = 255
@@ -205,8 +206,8 @@ def test_known_answer_clamp_and_bias(dev):
 
 def _sweep_cases(n=16, seed=2027):
     """Seeded random shapes: hidden and ispp multiples of 128 (stream kernels,
-    the last 256-k line zero-padded when not a multiple of 256) or of 32 (the
-    per-stage kernels), 1..300 tokens on 2..300 experts, bias and SwiGLU limit
+    the last 256-k line zero-padded when not a multiple of 256) or of 32 (odd
+    ones off the stream path), 1..300 tokens on 2..300 experts, bias and SwiGLU limit
     on or off."""
     import random
     rng = random.Random(seed)

@@ -13,8 +13,8 @@
 // (int4_stream.hip) into fp32 partial planes; mxfp4_swiglu_planes below finishes
 // stage 0 and the combine applies stage 1's roundings and bias. Every other
 // batch runs each stage through 32-row passes (mxfp4_stream_gemm below) or the
-// tile kernel (tile_gemm.hip), whichever its rows per expert and its number of
-// tiles make faster (capi.hip); both finish the stage in their epilogues. fp32
+// tile kernel (tile_gemm.hip), whichever its rows per expert, its contraction
+// and its number of tiles make faster (capi.hip); both finish the stage in their epilogues. fp32
 // activations are rounded to bf16 by the passes as they load them, before the
 // tile kernel.
 #include <algorithm>
@@ -31,8 +31,8 @@ namespace {
 // one 32-element e8m0 group of its weight row; a 32-row x 256-k activation chunk
 // is staged in LDS. Bound by latency (a chunk of loads in flight per wave) and,
 // from 33 rows per expert on, by reading the weights once per pass: E = 32,
-// hidden 2848, ispp 2912, top_k 4: 155 us at 16 tokens, 357 at 400, where the
-// tile kernel takes 214 and 268.
+// hidden 2848, ispp 2912, top_k 4: 155 us at 16 tokens, 357 at 400, where tiles
+// take about 180 and 255.
 constexpr int kChunkGroups = 8;           // 256 k per staged chunk
 constexpr int kChunkK = kChunkGroups * 32;
 constexpr int kRows = 32;                 // slots per pass (two MFMA row tiles)

@@ -44,9 +44,8 @@
 //
 // Measured per fused call against the kernels it replaces (MXFP4: 32-row passes
 // of a 4-wave workgroup per column block; INT4: the 256-row tile kernel): MXFP4
-// E = 256, hidden 4096, ispp 512, top_k 6, 4,096 tokens 1,190 -> 529 us; INT4
-// E = 48, N = 4096, K = 7168, top_k 8: 250 tokens 297 -> 256 us, 400 tokens 363
-// -> 285 us. At INT4, 4,096 tokens it draws the card's power limit (1.73 GHz at
+// E = 256, hidden 4096, ispp 512, top_k 6, 4,096 tokens 1,197 -> 468 us; INT4
+// E = 48, N = 4096, K = 7168, top_k 8, 250 tokens 297 -> 246 us. At INT4, 4,096 tokens it draws the card's power limit (1.73 GHz at
 // 59 % MFMA busy; builds without the activation loads, the dequant and the
 // weight loads run 265, 190 and 110 us faster).
 #include <algorithm>
