@@ -171,15 +171,16 @@ def select_backend(kernel_name: str, backend="auto") -> Backend:
         if want not in e.impls:
             raise _missing(kernel_name, want, e)
         return want
-    return _automatic(e)
+    return _automatic(e)[0]
 
 
-def _automatic(e: _Entry) -> Backend:
-    """The backend of ``backend="auto"`` with no environment override."""
+def _automatic(e: _Entry):
+    """The backend of ``backend="auto"`` with no environment override, and its callable."""
     for b in _PREFERENCE.get(detect_vendor(), (Backend.REFERENCE,)):
-        if b in e.impls:
-            return b
-    return next(iter(e.impls))
+        fn = e.impls.get(b)
+        if fn is not None:
+            return b, fn
+    return next(iter(e.impls.items()))
 
 
 def _warn_if_passed_over(kernel: str, chosen: Backend, args, kwargs) -> None:
@@ -205,11 +206,12 @@ def _warn_if_passed_over(kernel: str, chosen: Backend, args, kwargs) -> None:
 def dispatch(kernel_name: str, *args, backend="auto", **kwargs):
     """Runs ``kernel_name`` on the selected backend."""
     if backend == "auto" and not os.environ.get("XKERNELS_BACKEND", "").strip():
-        # select_backend without its second look at the environment (it raises the errors)
+        # select_backend's last rule without its second look at the environment
         e = _TABLE.get(kernel_name)
-        chosen = _automatic(e) if e is not None and e.impls else select_backend(kernel_name)
-        if chosen is Backend.REFERENCE:
-            _warn_if_passed_over(kernel_name, chosen, args, kwargs)
-    else:
-        chosen = select_backend(kernel_name, backend)
+        if e is not None and e.impls:
+            chosen, fn = _automatic(e)
+            if chosen is Backend.REFERENCE:
+                _warn_if_passed_over(kernel_name, chosen, args, kwargs)
+            return fn(*args, **kwargs)
+    chosen = select_backend(kernel_name, backend)
     return _TABLE[kernel_name].impls[chosen](*args, **kwargs)
