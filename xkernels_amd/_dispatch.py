@@ -171,16 +171,11 @@ def select_backend(kernel_name: str, backend="auto") -> Backend:
         if want not in e.impls:
             raise _missing(kernel_name, want, e)
         return want
-    return _automatic(e)[0]
-
-
-def _automatic(e: _Entry):
-    """The backend of ``backend="auto"`` with no environment override, and its callable."""
-    for b in _PREFERENCE.get(detect_vendor(), (Backend.REFERENCE,)):
-        fn = e.impls.get(b)
-        if fn is not None:
-            return b, fn
-    return next(iter(e.impls.items()))
+    order = _PREFERENCE.get(detect_vendor(), (Backend.REFERENCE,))
+    for b in order:
+        if b in e.impls:
+            return b
+    return next(iter(e.impls))
 
 
 def _warn_if_passed_over(kernel: str, chosen: Backend, args, kwargs) -> None:
@@ -206,12 +201,20 @@ def _warn_if_passed_over(kernel: str, chosen: Backend, args, kwargs) -> None:
 def dispatch(kernel_name: str, *args, backend="auto", **kwargs):
     """Runs ``kernel_name`` on the selected backend."""
     if backend == "auto" and not os.environ.get("XKERNELS_BACKEND", "").strip():
-        # select_backend's last rule without its second look at the environment
+        # an automatic choice, resolved here without a second look at the
+        # environment (select_backend's last rule, in line: a call to it costs the
+        # smallest ops 1-2 % of their 8 us; tests/test_host.py holds the two
+        # together; it also raises the errors)
         e = _TABLE.get(kernel_name)
         if e is not None and e.impls:
-            chosen, fn = _automatic(e)
-            if chosen is Backend.REFERENCE:
-                _warn_if_passed_over(kernel_name, chosen, args, kwargs)
-            return fn(*args, **kwargs)
-    chosen = select_backend(kernel_name, backend)
+            for b in _PREFERENCE.get(detect_vendor(), (Backend.REFERENCE,)):
+                fn = e.impls.get(b)
+                if fn is not None:
+                    if b is Backend.REFERENCE:
+                        _warn_if_passed_over(kernel_name, b, args, kwargs)
+                    return fn(*args, **kwargs)
+        chosen = select_backend(kernel_name, backend)
+        _warn_if_passed_over(kernel_name, chosen, args, kwargs)
+    else:
+        chosen = select_backend(kernel_name, backend)
     return _TABLE[kernel_name].impls[chosen](*args, **kwargs)
