@@ -202,8 +202,7 @@ def dispatch(kernel_name: str, *args, backend="auto", **kwargs):
     """Runs ``kernel_name`` on the selected backend."""
     if backend == "auto" and not os.environ.get("XKERNELS_BACKEND", "").strip():
         # an automatic choice, resolved here without a second look at the
-        # environment (select_backend's last rule, in line: a call to it costs the
-        # smallest ops 1-2 % of their 8 us; tests/test_host.py holds the two
+        # environment (select_backend's last rule in line; a test holds the two
         # together; it also raises the errors)
         e = _TABLE.get(kernel_name)
         if e is not None and e.impls:
