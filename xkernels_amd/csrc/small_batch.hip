@@ -391,7 +391,8 @@ bool small_int4_faster(int64_t M, int64_t top_k, int64_t E, int64_t routed, int6
   const double k1 = double(K) / 1e3, all = experts * double(N) * double(K) / 1e7;
   const int64_t cus = device_cu_count(), per_cu = cdiv(N / 16, cus);
   const bool alone = per_cu > 1 && row_lds(M, K) + kStaticLds > kTwoWorkgroupLds;
-  const double here = 5.0 + 0.09 * experts + k1 * (experts * double(per_cu) * (alone ? 0.46 : 0.3) + 0.085 * double(M)) + 0.3 * all;
+  const double walk = experts * double(per_cu) * (alone ? 0.46 : 0.3) + 0.085 * double(M);
+  const double here = 5.0 + 0.09 * experts + k1 * walk + 0.3 * all;
   const double stream = 10.5 + 0.1 * experts + k1 + 0.89 * all + 1.5e-6 * double(M * top_k) * double(N);
   return here < stream;
 }

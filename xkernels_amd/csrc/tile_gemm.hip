@@ -38,16 +38,17 @@
 //     to 128 tiles measured the same). The XCDs' counters sit a cache line apart
 //     where the caller's buffer allows: atomics on one line wait for each other
 //     over all XCDs, which cost a launch about 25 us (gate/up of E = 64, hidden
-//     256, ispp 2048, 30 rows per expert, 1,024 tiles, per call: 105 -> 80 us). Tiles that
-//     all fit the places at once are dealt without the queue (E = 64, hidden =
-//     ispp = 256, 448 tokens, top_k 4, per call: 72 -> 36 us).
+//     256, ispp 2048, 30 rows per expert, 1,024 tiles, per call: 105 -> 80 us).
+//     Tiles that all fit the places at once are dealt without the queue (E = 64,
+//     hidden = ispp = 256, 448 tokens, top_k 4, per call: 72 -> 36 us).
 //
 // Measured per fused call against the kernels it replaces (MXFP4: 32-row passes
 // of a 4-wave workgroup per column block; INT4: the 256-row tile kernel): MXFP4
 // E = 256, hidden 4096, ispp 512, top_k 6, 4,096 tokens 1,197 -> 468 us; INT4
-// E = 48, N = 4096, K = 7168, top_k 8, 250 tokens 297 -> 246 us. At INT4, 4,096 tokens it draws the card's power limit (1.73 GHz at
-// 59 % MFMA busy; builds without the activation loads, the dequant and the
-// weight loads run 265, 190 and 110 us faster).
+// E = 48, N = 4096, K = 7168, top_k 8, 250 tokens 297 -> 246 us. At INT4, 4,096
+// tokens it draws the card's power limit (1.73 GHz at 59 % MFMA busy; builds
+// without the activation loads, the dequant and the weight loads run 265, 190 and
+// 110 us faster).
 #include <algorithm>
 #include <type_traits>
 
